@@ -675,9 +675,24 @@ static hipError_t launch_dec(const float* x, const uint8_t* w, size_t row_bytes,
     return hipGetLastError();
 }
 
+// The per-lane form: any row length, and no byte past a row's end is read.
+static hipError_t launch_per_lane(CanonFormat fmt, const float* x, const uint8_t* w, size_t row_bytes, float* y, int batch,
+                                  int in_feat, int out_feat, hipStream_t stream) {
+    switch (fmt) {
+    case kCanonQ8_0: return launch_dec<DecQ8_0>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
+    case kCanonQ5_0: return launch_dec<DecQ5_0>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
+    case kCanonQ4_0: return launch_dec<DecQ4_0>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
+    case kCanonF32: return launch_dec<DecF32>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
+    case kCanonQ4KFloat: return launch_dec<DecQ4KFloat>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_canon_gemv(CanonFormat fmt, const float* x, const uint8_t* w, size_t row_bytes, float* y,
                              int batch, int in_feat, int out_feat, int num_cus, hipStream_t stream) {
     (void)num_cus;
+    if (canon_gemm_faster(fmt, batch, in_feat, out_feat))
+        return launch_canon_gemm(fmt, x, w, row_bytes, y, batch, in_feat, out_feat, stream);
     if (in_feat % 4 == 0) {  // windowed form: x rows stay float4-aligned
         switch (fmt) {
         case kCanonQ8_0:
@@ -691,14 +706,7 @@ hipError_t launch_canon_gemv(CanonFormat fmt, const float* x, const uint8_t* w, 
         }
         return hipErrorInvalidValue;
     }
-    switch (fmt) {  // per-lane form (f32 rows whose length is not a multiple of 4)
-    case kCanonQ8_0: return launch_dec<DecQ8_0>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
-    case kCanonQ5_0: return launch_dec<DecQ5_0>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
-    case kCanonQ4_0: return launch_dec<DecQ4_0>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
-    case kCanonF32: return launch_dec<DecF32>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
-    case kCanonQ4KFloat: return launch_dec<DecQ4KFloat>(x, w, row_bytes, y, batch, in_feat, out_feat, stream);
-    }
-    return hipErrorInvalidValue;
+    return launch_per_lane(fmt, x, w, row_bytes, y, batch, in_feat, out_feat, stream);
 }
 
 int canon_max_in_feat() { return kMaxChunkSlots * kChunk; }
@@ -717,8 +725,8 @@ hipError_t launch_canon_segment(CanonFormat fmt, const float* x, const uint8_t* 
         }
         return hipErrorInvalidValue;
     }
-    // the per-lane form reads only inside each row's segment
-    return launch_canon_gemv(fmt, x, w, row_bytes, y, batch, seg_in, out_feat, 0, stream);
+    // f32 rows whose length is not a multiple of 4
+    return launch_per_lane(fmt, x, w, row_bytes, y, batch, seg_in, out_feat, stream);
 }
 
 __global__ void fill_kernel(float* __restrict__ y, size_t n, float v) {
