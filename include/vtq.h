@@ -142,12 +142,12 @@ int vtq_linear_device(vtq_ctx *ctx, int ggml_type, int regime, const float *d_x,
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same computation, arguments and
  * errors as vtq_linear_device, but it calls no hipMalloc / hipFree: the
- * prefill GEMM's workspace (the quantized activations, batch >= 32 on Q4_K
- * in the integer regime) lives in a fixed 32 MiB array on each GPU,
- * allocated when the library loads.  Requests whose workspace would exceed
- * it (vtq::q4k_gemm_workspace_bytes: about batch x in_feat x 1.14 bytes,
- * batch capped at 8192 per chunk) return VTQ_E_NOT_IMPLEMENTED with a
- * message and launch nothing.  Rows longer than the kernels hold (k-quant
+ * batch GEMM's workspace (the quantized activations; Q4_K in the integer
+ * regime and Q6_K, batch > 2) lives in a fixed 32 MiB array on each GPU,
+ * allocated when the library loads.  Q4_K requests whose workspace would
+ * exceed it (vtq::q4k_gemm_workspace_bytes: about batch x in_feat x 1.14
+ * bytes, batch capped at 8192 per chunk) return VTQ_E_NOT_IMPLEMENTED with a
+ * message and launch nothing; Q6_K walks the batch in chunks that fit.  Rows longer than the kernels hold (k-quant
  * beyond 32768 inputs, the canonical dot beyond 65536) keep their
  * segments' sums there too (segments x batch x out_feat x 4 bytes, plus one
  * gathered segment of x per batch row for the canonical dot), with the

@@ -1,6 +1,7 @@
-// q4k_gemm.hip -- exact-integer Q4_K prefill GEMM on i8 MFMA (gfx950).
+// q4k_gemm.hip -- exact-integer Q4_K and Q6_K batch GEMM on i8 MFMA (gfx950).
 //
-// Replaces linear_q4_k_integer (src/ops/quant.rs:936-980) for large batch:
+// Replaces linear_q4_k_integer (src/ops/quant.rs:936-980) and, in the split-K
+// kernel, linear_q6_k_integer (:1060-1096) for batches.  Q4_K:
 // y[b][o] = fixed_tree_s part(b, o, s) with, per super-block s,
 //   acc  = sum_j sc_j * sum_{k in j} q_k * xq_k          (j = 8 sub-blocks of 32)
 //   accm = sum_j m_j  * bsum_j
@@ -81,9 +82,10 @@ inline GemmWs gemm_ws(void* base, int Mp, int R) {
 // Workgroup (s, q) holds the 16 consecutive tokens 16q..16q+15 of
 // super-block s, so each 256-byte run of the token operands (and the 16
 // d / bsum entries beside it) is written by one workgroup at once.
+enum MinTerm { kMinI8 = 0, kMinF16 = 1, kMinNone = 2 };
 constexpr int kQuantWaves = 16;
 __global__ __launch_bounds__(kQuantWaves * 64) void act_quant_tiles_kernel(const float* __restrict__ x, GemmWs ws,
-                                                                           int R, int M, int f16_min) {
+                                                                           int R, int M, int min_term) {
     const int lane = threadIdx.x & 63;
     const int s = (int)blockIdx.x;
     const int b = (int)blockIdx.y * kQuantWaves + wave_id();  // < Mp: the grid covers Mp / 16 groups
@@ -101,8 +103,8 @@ __global__ __launch_bounds__(kQuantWaves * 64) void act_quant_tiles_kernel(const
     uint8_t* dst = reinterpret_cast<uint8_t*>(ws.xqt + ((size_t)tile * 8 + j) * 64 + 32 * g + n) + 4 * (lane & 3);
     *reinterpret_cast<uint32_t*>(dst) = packed;
     if (lane == 0) ws.xdt[(size_t)tile * 32 + n] = d;
-    if ((lane & 7) == 0) {
-        if (f16_min) {
+    if ((lane & 7) == 0 && min_term != kMinNone) {
+        if (min_term == kMinF16) {
             // exact in f16: |64*bh| <= 4096 is a multiple of 64, 0 <= bl <= 63
             _Float16* o = reinterpret_cast<_Float16*>(ws.xmt + (size_t)tile * 64 + n);
             o[j] = (_Float16)(float)(s32 - (s32 & 63));  // 64*bh
@@ -377,124 +379,13 @@ __device__ __forceinline__ uint32_t pk_f16(uint32_t a, uint32_t b) {  // two sma
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz((float)a, (float)b));
 }
 
-// The per-wave work: rows o0 .. o0+31 and token tiles NT*tp .. NT*tp+NT-1,
-// the parts of super-blocks s0 .. s0+Rl-1 folded by fixed_tree over those Rl
-// leaves into res (the row's result when s0 = 0 and Rl = R; the value of one
-// subtree when Rl is a power of two and s0 a multiple of it).  Rl <= 16.
-// lv: this wave's LDS tree levels 2 and 3; dd: its d / dmin slots.
-template <int NT>
-__device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const GemmWs& ws, int R, int N, int M, int o0,
-                                        int tp, int s0, int Rl, float4* lv, float* dd, float (&res)[NT][16]) {
-    constexpr int D = 4;  // k-steps of token operands in flight
+// fixed_tree over a wave's Rl leaves into res: sblock(s, p) gives leaf s of
+// every tile.  Levels 0 and 1 of the counter stay in registers, levels 2 and
+// 3 in the wave's own LDS (lv; only for Rl > 4 and Rl > 8).
+template <int NT, class SB>
+__device__ __forceinline__ void fold_leaves(int Rl, float4* lv, float (&res)[NT][16], SB&& sblock) {
     const int lane = threadIdx.x & 63;
-    const int r = lane & 31, g = lane >> 5;
-    const int Mt = (M + 31) / 32;
-
-    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(ws.xqt, (short)0, Mt * R * 8192, kGemmWord3);
-    const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(ws.xmt, (short)0, Mt * R * 1024, kGemmWord3);
-    const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(ws.xdt, (short)0, Mt * R * 128, kGemmWord3);
-    const __amdgpu_buffer_rsrc_t rw =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(W), (short)0, N * R * 144, kGemmWord3);
-    uint32_t q0[NT], m0[NT], d0[NT];  // tile bases (scalar); past the end a tile recomputes the last one
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const uint32_t T = (uint32_t)min(NT * tp + t, Mt - 1);
-        q0[t] = (T * R + s0) * 8192;
-        m0[t] = (T * R + s0) * 1024;
-        d0[t] = (T * R + s0) * 128;
-    }
-    const uint32_t vq = 16u * lane, vd = 4u * r;
-    // lane (r, g): header of row r, and code bytes 32h + 16g .. +15 of each
-    // quarter h: low nibbles are k-step 2h, high nibbles k-step 2h + 1, both
-    // at k = 16g .. 16g + 15 of the step (the B operand's order)
-    const uint32_t vh = (uint32_t)min(o0 + r, N - 1) * ((uint32_t)R * 144) + (uint32_t)s0 * 144, vc = vh + 16 + 16 * g;
-
-    uint4 hdr = __builtin_bit_cast(uint4, bload16(rw, vh, 0));
-    uint4 qw[4];
-#pragma unroll
-    for (int h = 0; h < 4; h++) qw[h] = __builtin_bit_cast(uint4, bload16(rw, vc + 32 * h, 0));
-    v4i bq[NT][D];  // token operands: ring of D k-steps
-#pragma unroll
-    for (int j = 0; j < D; j++)
-#pragma unroll
-        for (int t = 0; t < NT; t++) bq[t][j] = bload16(rq, vq, q0[t] + j * 1024);
-    v4i bm[NT];
-    float dx[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        bm[t] = bload16(rm, vq, m0[t]);
-        dx[t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t], 0));
-    }
-
     float L0[NT][16], L1[NT][16];
-
-    // one super-block: the parts of every tile into p
-    auto sblock = [&](int s, float (&p)[NT][16]) __attribute__((always_inline)) {
-        const int sn = min(s + 1, Rl - 1);
-        // get_scale_min_k4 (src/ops/quant.rs:267-276) of all eight sub-blocks, a byte each
-        const uint32_t Y = hdr.y, Z = hdr.z, Wd = hdr.w;
-        const uint32_t SCl = Y & 0x3F3F3F3Fu, Ml = Z & 0x3F3F3F3Fu;
-        const uint32_t SCh = (Wd & 0x0F0F0F0Fu) | ((Y >> 2) & 0x30303030u);
-        const uint32_t Mh = ((Wd >> 4) & 0x0F0F0F0Fu) | ((Z >> 2) & 0x30303030u);
-        const uint32_t SHl = (SCl >> 3) & 0x07070707u, SLl = SCl & 0x07070707u;
-        const uint32_t SHh = (SCh >> 3) & 0x07070707u, SLh = SCh & 0x07070707u;
-        if (g == 0) {
-            dd[r] = f16_to_f32_sel(hdr.x & 0xFFFFu);
-            dd[32 + r] = f16_to_f32_sel(hdr.x >> 16);
-        }
-        const uint32_t am0 = pk_f16(Ml & 255u, (Ml >> 8) & 255u), am1 = pk_f16((Ml >> 16) & 255u, Ml >> 24);
-        const uint32_t am2 = pk_f16(Mh & 255u, (Mh >> 8) & 255u), am3 = pk_f16((Mh >> 16) & 255u, Mh >> 24);
-        const v8h am = __builtin_bit_cast(v8h, v4i{(int)am0, (int)am1, (int)am2, (int)am3});
-        hdr = __builtin_bit_cast(uint4, bload16(rw, vh, (uint32_t)sn * 144));
-        v16i c1[NT], c0[NT];
-#pragma unroll
-        for (int t = 0; t < NT; t++) c1[t] = c0[t] = v16i{};
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int h = j >> 1, sh = 4 * (j & 1);
-            const uint32_t SH = j < 4 ? SHl : SHh, SL = j < 4 ? SLl : SLh;
-            const us2 mh = __builtin_bit_cast(us2, rep_byte16(SH, j & 3));
-            const us2 ml = __builtin_bit_cast(us2, rep_byte16(SL, j & 3));
-            const uint32_t w0 = (qw[h].x >> sh) & 0x0F0F0F0Fu, w1 = (qw[h].y >> sh) & 0x0F0F0F0Fu;
-            const uint32_t w2 = (qw[h].z >> sh) & 0x0F0F0F0Fu, w3 = (qw[h].w >> sh) & 0x0F0F0F0Fu;
-            const v4i a1 = v4i{nib_mul(w0, mh), nib_mul(w1, mh), nib_mul(w2, mh), nib_mul(w3, mh)};
-            const v4i a0 = v4i{nib_mul(w0, ml), nib_mul(w1, ml), nib_mul(w2, ml), nib_mul(w3, ml)};
-            if (j & 1) qw[h] = __builtin_bit_cast(uint4, bload16(rw, vc + 32 * h, (uint32_t)sn * 144));
-#pragma unroll
-            for (int t = 0; t < NT; t++) c1[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bq[t][j % D], c1[t], 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < NT; t++) c0[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bq[t][j % D], c0[t], 0, 0, 0);
-            // refill the ring slot: k-step j + D of this super-block, or of the next
-            const uint32_t kk = (uint32_t)(j + D < 8 ? s * 8 + j + D : sn * 8 + j + D - 8) * 1024;
-#pragma unroll
-            for (int t = 0; t < NT; t++) bq[t][j % D] = bload16(rq, vq, q0[t] + kk);
-        }
-        // min term (src/ops/quant.rs:876-883): accm = sum_j m_j * bsum_j
-        v16f cm[NT];
-        float ds[NT];
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            cm[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, __builtin_bit_cast(v8h, bm[t]), v16f{}, 0, 0, 0);
-            ds[t] = dx[t];
-            bm[t] = bload16(rm, vq, m0[t] + (uint32_t)sn * 1024);
-            dx[t] = __builtin_bit_cast(float,
-                                       __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t] + (uint32_t)sn * 128, 0));
-        }
-        // epilogue (src/ops/quant.rs:849-898): element i of a lane is row 8*(i/4) + 4*g + i%4, token r
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float4 dv = *reinterpret_cast<const float4*>(dd + 8 * q + 4 * g);
-            const float4 mv = *reinterpret_cast<const float4*>(dd + 32 + 8 * q + 4 * g);
-            const float dr[4] = {dv.x, dv.y, dv.z, dv.w}, mr[4] = {mv.x, mv.y, mv.z, mv.w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int i = 4 * q + e;
-#pragma unroll
-                for (int t = 0; t < NT; t++)
-                    p[t][i] = ((dr[e] * ds[t]) * (float)(8 * c1[t][i] + c0[t][i])) - ((mr[e] * ds[t]) * cm[t][i]);
-            }
-        }
-    };
     auto lds_store = [&](int l, const float (&v)[NT][16]) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NT; t++)
@@ -566,6 +457,268 @@ __device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const Gem
         if (L < 2 && ((Rl >> 2) & 1)) lds_merge(2, res);
         if (L < 3 && ((Rl >> 3) & 1)) lds_merge(3, res);
     }
+}
+
+// The per-wave work: rows o0 .. o0+31 and token tiles NT*tp .. NT*tp+NT-1,
+// the parts of super-blocks s0 .. s0+Rl-1 folded by fixed_tree over those Rl
+// leaves into res (the row's result when s0 = 0 and Rl = R; the value of one
+// subtree when Rl is a power of two and s0 a multiple of it).  Rl <= 16.
+// lv: this wave's LDS tree levels 2 and 3; dd: its d / dmin slots.
+template <int NT>
+__device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const GemmWs& ws, int R, int N, int M, int o0,
+                                        int tp, int s0, int Rl, float4* lv, float* dd, float (&res)[NT][16]) {
+    constexpr int D = 4;  // k-steps of token operands in flight
+    const int lane = threadIdx.x & 63;
+    const int r = lane & 31, g = lane >> 5;
+    const int Mt = (M + 31) / 32;
+
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(ws.xqt, (short)0, Mt * R * 8192, kGemmWord3);
+    const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(ws.xmt, (short)0, Mt * R * 1024, kGemmWord3);
+    const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(ws.xdt, (short)0, Mt * R * 128, kGemmWord3);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(W), (short)0, N * R * 144, kGemmWord3);
+    uint32_t q0[NT], m0[NT], d0[NT];  // tile bases (scalar); past the end a tile recomputes the last one
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const uint32_t T = (uint32_t)min(NT * tp + t, Mt - 1);
+        q0[t] = (T * R + s0) * 8192;
+        m0[t] = (T * R + s0) * 1024;
+        d0[t] = (T * R + s0) * 128;
+    }
+    const uint32_t vq = 16u * lane, vd = 4u * r;
+    // lane (r, g): header of row r, and code bytes 32h + 16g .. +15 of each
+    // quarter h: low nibbles are k-step 2h, high nibbles k-step 2h + 1, both
+    // at k = 16g .. 16g + 15 of the step (the B operand's order)
+    const uint32_t vh = (uint32_t)min(o0 + r, N - 1) * ((uint32_t)R * 144) + (uint32_t)s0 * 144, vc = vh + 16 + 16 * g;
+
+    uint4 hdr = __builtin_bit_cast(uint4, bload16(rw, vh, 0));
+    uint4 qw[4];
+#pragma unroll
+    for (int h = 0; h < 4; h++) qw[h] = __builtin_bit_cast(uint4, bload16(rw, vc + 32 * h, 0));
+    v4i bq[NT][D];  // token operands: ring of D k-steps
+#pragma unroll
+    for (int j = 0; j < D; j++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) bq[t][j] = bload16(rq, vq, q0[t] + j * 1024);
+    v4i bm[NT];
+    float dx[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        bm[t] = bload16(rm, vq, m0[t]);
+        dx[t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t], 0));
+    }
+
+    // one super-block: the parts of every tile into p
+    auto sblock = [&](int s, float (&p)[NT][16]) __attribute__((always_inline)) {
+        const int sn = min(s + 1, Rl - 1);
+        // get_scale_min_k4 (src/ops/quant.rs:267-276) of all eight sub-blocks, a byte each
+        const uint32_t Y = hdr.y, Z = hdr.z, Wd = hdr.w;
+        const uint32_t SCl = Y & 0x3F3F3F3Fu, Ml = Z & 0x3F3F3F3Fu;
+        const uint32_t SCh = (Wd & 0x0F0F0F0Fu) | ((Y >> 2) & 0x30303030u);
+        const uint32_t Mh = ((Wd >> 4) & 0x0F0F0F0Fu) | ((Z >> 2) & 0x30303030u);
+        const uint32_t SHl = (SCl >> 3) & 0x07070707u, SLl = SCl & 0x07070707u;
+        const uint32_t SHh = (SCh >> 3) & 0x07070707u, SLh = SCh & 0x07070707u;
+        if (g == 0) {
+            dd[r] = f16_to_f32_sel(hdr.x & 0xFFFFu);
+            dd[32 + r] = f16_to_f32_sel(hdr.x >> 16);
+        }
+        const uint32_t am0 = pk_f16(Ml & 255u, (Ml >> 8) & 255u), am1 = pk_f16((Ml >> 16) & 255u, Ml >> 24);
+        const uint32_t am2 = pk_f16(Mh & 255u, (Mh >> 8) & 255u), am3 = pk_f16((Mh >> 16) & 255u, Mh >> 24);
+        const v8h am = __builtin_bit_cast(v8h, v4i{(int)am0, (int)am1, (int)am2, (int)am3});
+        hdr = __builtin_bit_cast(uint4, bload16(rw, vh, (uint32_t)sn * 144));
+        v16i c1[NT], c0[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) c1[t] = c0[t] = v16i{};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int h = j >> 1, sh = 4 * (j & 1);
+            const uint32_t SH = j < 4 ? SHl : SHh, SL = j < 4 ? SLl : SLh;
+            const us2 mh = __builtin_bit_cast(us2, rep_byte16(SH, j & 3));
+            const us2 ml = __builtin_bit_cast(us2, rep_byte16(SL, j & 3));
+            const uint32_t w0 = (qw[h].x >> sh) & 0x0F0F0F0Fu, w1 = (qw[h].y >> sh) & 0x0F0F0F0Fu;
+            const uint32_t w2 = (qw[h].z >> sh) & 0x0F0F0F0Fu, w3 = (qw[h].w >> sh) & 0x0F0F0F0Fu;
+            const v4i a1 = v4i{nib_mul(w0, mh), nib_mul(w1, mh), nib_mul(w2, mh), nib_mul(w3, mh)};
+            const v4i a0 = v4i{nib_mul(w0, ml), nib_mul(w1, ml), nib_mul(w2, ml), nib_mul(w3, ml)};
+            if (j & 1) qw[h] = __builtin_bit_cast(uint4, bload16(rw, vc + 32 * h, (uint32_t)sn * 144));
+#pragma unroll
+            for (int t = 0; t < NT; t++) c1[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bq[t][j % D], c1[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < NT; t++) c0[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bq[t][j % D], c0[t], 0, 0, 0);
+            // refill the ring slot: k-step j + D of this super-block, or of the next
+            const uint32_t kk = (uint32_t)(j + D < 8 ? s * 8 + j + D : sn * 8 + j + D - 8) * 1024;
+#pragma unroll
+            for (int t = 0; t < NT; t++) bq[t][j % D] = bload16(rq, vq, q0[t] + kk);
+        }
+        // min term (src/ops/quant.rs:876-883): accm = sum_j m_j * bsum_j
+        v16f cm[NT];
+        float ds[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            cm[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, __builtin_bit_cast(v8h, bm[t]), v16f{}, 0, 0, 0);
+            ds[t] = dx[t];
+            bm[t] = bload16(rm, vq, m0[t] + (uint32_t)sn * 1024);
+            dx[t] = __builtin_bit_cast(float,
+                                       __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t] + (uint32_t)sn * 128, 0));
+        }
+        // epilogue (src/ops/quant.rs:849-898): element i of a lane is row 8*(i/4) + 4*g + i%4, token r
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 dv = *reinterpret_cast<const float4*>(dd + 8 * q + 4 * g);
+            const float4 mv = *reinterpret_cast<const float4*>(dd + 32 + 8 * q + 4 * g);
+            const float dr[4] = {dv.x, dv.y, dv.z, dv.w}, mr[4] = {mv.x, mv.y, mv.z, mv.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int i = 4 * q + e;
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    p[t][i] = ((dr[e] * ds[t]) * (float)(8 * c1[t][i] + c0[t][i])) - ((mr[e] * ds[t]) * cm[t][i]);
+            }
+        }
+    };
+    fold_leaves<NT>(Rl, lv, res, sblock);
+}
+
+// The same for Q6_K rows (dot_q6k_q8_block, src/ops/quant.rs:995-1057): 16
+// sub-blocks of 16 codes c = code - 32 with a signed 8-bit scale sc each.
+//   acc  = sum_i sc_i * sum_{k in i} c_k * xq_k,   part = (d*dx) * f32(acc)
+// The scale is folded into the operand: v = c*sc (13 bits signed) as two
+// signed bytes, v = 256*hi + lo with lo the low byte read as i8 and hi = (v +
+// 128) >> 8, so acc = 256*C1 + C0 from 16 i8 MFMAs (|lo| <= 128, |hi| <= 16;
+// |acc| <= 256*32*128*127 < 2^31).  The products are formed two to a register
+// with 16-bit multiply-adds, code*sc + (128 - 32*sc) = v + 128, whose high
+// bytes are hi and whose low bytes are lo + 128 (mod 256): about 350 vector
+// instructions a super-block, shared by the wave's token tiles.
+template <int NT>
+__device__ __forceinline__ void pw6_tree(const uint8_t* __restrict__ W, const GemmWs& ws, int R, int N, int M, int o0,
+                                         int tp, int s0, int Rl, float4* lv, v4i* stage, float* dd,
+                                         float (&res)[NT][16]) {
+    constexpr int D = 4;  // k-steps of token operands in flight
+    const int lane = threadIdx.x & 63;
+    const int r = lane & 31, g = lane >> 5;
+    const int Mt = (M + 31) / 32;
+
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(ws.xqt, (short)0, Mt * R * 8192, kGemmWord3);
+    const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(ws.xdt, (short)0, Mt * R * 128, kGemmWord3);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(W), (short)0, N * R * 210, kGemmWord3);
+    uint32_t q0[NT], d0[NT];  // tile bases (scalar); past the end a tile recomputes the last one
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const uint32_t T = (uint32_t)min(NT * tp + t, Mt - 1);
+        q0[t] = (T * R + s0) * 8192;
+        d0[t] = (T * R + s0) * 128;
+    }
+    const uint32_t vq = 16u * lane, vd = 4u * r;
+    // Weights.  The first 208 bytes of each row's block (128 low-bit bytes, 64
+    // high-bit bytes, 16 scales) are 13 chunks of 16; load k of lane L takes
+    // chunk 64k + L of the 32 rows' 416, so a load covers 208 contiguous bytes
+    // of every row it touches, and the wave's LDS holds the rows 208 bytes
+    // apart (13 chunks, odd: the row-per-lane reads below meet in no bank).
+    // Read straight into the lanes that use them, each at its own row, they
+    // cost 2022 cache accesses a super-block instead of 727 and the 200-token
+    // case above 135 us.  (Aligned chunks, moved into place by unaligned LDS
+    // writes, cost 306 accesses but 106.7 us: such writes are slow.)
+    constexpr int kCh = 13, kLoads = 7;
+    const uint32_t row_bytes = (uint32_t)R * 210;
+    uint32_t vw[kLoads];
+#pragma unroll
+    for (int k = 0; k < kLoads; k++) {
+        const int i = min(64 * k + lane, 32 * kCh - 1);  // past the last chunk: not stored
+        vw[k] = (uint32_t)min(o0 + i / kCh, N - 1) * row_bytes + (uint32_t)s0 * 210 + 16u * (uint32_t)(i % kCh);
+    }
+    const uint32_t vd0 = (uint32_t)min(o0 + r, N - 1) * row_bytes + (uint32_t)s0 * 210 + 208;
+    v4i wt[kLoads];
+    uint32_t dh;
+    auto wload = [&](uint32_t so) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kLoads; k++) wt[k] = bload16(rw, vw[k], so);
+        dh = __builtin_amdgcn_raw_buffer_load_b16(rw, vd0, so, 0);
+    };
+    // lane (r, g) holds positions 16g .. 16g+15 of every run of 32: low-bit
+    // bytes 64h + 32b + 16g .. +15, high-bit bytes 128 + 32h + 16g .. +15 of
+    // half h; k-step 4h + q takes b = q & 1 (low nibbles for q < 2) and bits
+    // 2q, 2q + 1, at scale 8h + 2q + g
+    const v4i* wrow = stage + kCh * r;
+    wload(0);
+    __builtin_amdgcn_sched_barrier(0);
+    v4i bq[NT][D];  // token operands: ring of D k-steps
+#pragma unroll
+    for (int j = 0; j < D; j++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) bq[t][j] = bload16(rq, vq, q0[t] + j * 1024);
+
+    auto sblock = [&](int s, float (&p)[NT][16]) __attribute__((always_inline)) {
+        const int sn = min(s + 1, Rl - 1);
+#pragma unroll
+        for (int k = 0; k < kLoads; k++)
+            if (k + 1 < kLoads || lane < 32 * kCh - 64 * (kLoads - 1)) stage[64 * k + lane] = wt[k];
+        if (g == 0) dd[r] = f16_hw(dh);
+        // this super-block's token scales: loads complete in order, so they go
+        // before the next weights, which nothing here may wait for
+        float ds[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            ds[t] = __builtin_bit_cast(float,
+                                       __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t] + (uint32_t)s * 128, 0));
+        const v4i sc = wrow[12];
+        uint32_t sw[4];  // scale bytes 2m + g at the even bytes
+#pragma unroll
+        for (int k = 0; k < 4; k++) sw[k] = (uint32_t)sc[k] >> (8 * g);
+        v16i c1[NT], c0[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) c1[t] = c0[t] = v16i{};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int h = j >> 2, q = j & 3;
+            const v4i ql = wrow[4 * h + 2 * (q & 1) + g], qh = wrow[8 + 2 * h + g];
+            const int scj = (int)(int8_t)(uint8_t)(sw[j >> 1] >> (16 * (j & 1)));
+            const us2 ms = {(unsigned short)scj, (unsigned short)scj};
+            const us2 mo = {(unsigned short)(128 - 32 * scj), (unsigned short)(128 - 32 * scj)};
+            v4i a1, a0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t n = ((uint32_t)ql[e] >> (q < 2 ? 0 : 4)) & 0x0F0F0F0Fu;
+                const uint32_t b = (uint32_t)qh[e];
+                const uint32_t c = n | (q == 0   ? (b & 0x03030303u) << 4
+                                        : q == 1 ? (b & 0x0C0C0C0Cu) << 2
+                                        : q == 2 ? b & 0x30303030u
+                                                 : (b >> 2) & 0x30303030u);
+                const us2 ve = __builtin_bit_cast(us2, c & 0x00FF00FFu) * ms + mo;
+                const us2 vo = __builtin_bit_cast(us2, (c >> 8) & 0x00FF00FFu) * ms + mo;
+                const uint32_t we = __builtin_bit_cast(uint32_t, ve), wo = __builtin_bit_cast(uint32_t, vo);
+                a1[e] = (int)__builtin_amdgcn_perm(wo, we, 0x07030501u);
+                a0[e] = (int)(__builtin_amdgcn_perm(wo, we, 0x06020400u) ^ 0x80808080u);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; t++) c1[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bq[t][j % D], c1[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < NT; t++) c0[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bq[t][j % D], c0[t], 0, 0, 0);
+            // refill the ring slot: k-step j + D of this super-block, or of the next
+            const uint32_t kk = (uint32_t)(j + D < 8 ? s * 8 + j + D : sn * 8 + j + D - 8) * 1024;
+#pragma unroll
+            for (int t = 0; t < NT; t++) bq[t][j % D] = bload16(rq, vq, q0[t] + kk);
+            if (j == D - 1) {
+                // the next super-block's weights, behind the last token
+                // operands that this one still uses
+                __builtin_amdgcn_sched_barrier(0);
+                wload((uint32_t)sn * 210);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // element i of a lane is row 8*(i/4) + 4*g + i%4, token r
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 dv = *reinterpret_cast<const float4*>(dd + 8 * q + 4 * g);
+            const float dr[4] = {dv.x, dv.y, dv.z, dv.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int i = 4 * q + e;
+#pragma unroll
+                for (int t = 0; t < NT; t++) p[t][i] = (dr[e] * ds[t]) * (float)(256 * c1[t][i] + c0[t][i]);
+            }
+        }
+    };
+    fold_leaves<NT>(Rl, lv, res, sblock);
 }
 
 template <int NT>
@@ -654,15 +807,27 @@ static int sk_piece(int R, int T) {
     return first;
 }
 
+constexpr int kQ6StageBytes = 32 * 208;
+__host__ __device__ constexpr int sk_lds_per_wave(bool q6, int C) {
+    return (q6 ? kQ6StageBytes + 128 : 4096 + 256) + (C > 8 ? 2 : C > 4 ? 1 : 0) * pw_level_bytes(1);
+}
+
+template <bool Q6>
 __global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const uint8_t* __restrict__ W, GemmWs ws,
                                                                            float* __restrict__ y, int R, int N, int M,
                                                                            int C) {
-    constexpr int kW = pw_lds_per_wave(1);
     extern __shared__ __align__(16) unsigned char lds[];
-    const int lane = threadIdx.x & 63, wave = wave_id(), nw = (int)(blockDim.x >> 6);
-    float4* lv = reinterpret_cast<float4*>(lds + (size_t)wave * kW);
-    float* dd = reinterpret_cast<float*>(lds + (size_t)wave * kW + 2 * pw_level_bytes(1));
-    float4* cv = reinterpret_cast<float4*>(lds + (size_t)nw * kW);  // [chunk][q][lane]
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    // per wave: the Q6_K weight stage, in which its chunk's value goes once
+    // the chunk is folded, or (Q4_K) a place for that value; then d of the
+    // rows (Q4_K: and dmin); then tree level 2 for pieces of more than 4
+    // leaves and level 3 for more than 8
+    const int kW = sk_lds_per_wave(Q6, C);
+    constexpr int kVal = Q6 ? kQ6StageBytes : 4096, kDd = Q6 ? 128 : 256;
+    unsigned char* const base = lds + (size_t)wave * kW;
+    float* dd = reinterpret_cast<float*>(base + kVal);
+    float4* lv = reinterpret_cast<float4*>(base + kVal + kDd);
+    auto cv = [&](int c) { return reinterpret_cast<float4*>(lds + (size_t)c * kW); };  // [q][lane] of chunk c
     const int Mt = (M + 31) / 32, rt = (int)blockIdx.x / Mt, tt = (int)blockIdx.x % Mt;
     const int r = lane & 31, g = lane >> 5;
     // this wave's chunk
@@ -682,10 +847,13 @@ __global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const 
         }
     }
     float res[1][16];
-    pw_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, dd, res);
+    if constexpr (Q6)
+        pw6_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, reinterpret_cast<v4i*>(base), dd, res);
+    else
+        pw_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, dd, res);
 #pragma unroll
     for (int q = 0; q < 4; q++)
-        cv[(wave * 4 + q) * 64 + lane] = make_float4(res[0][4 * q], res[0][4 * q + 1], res[0][4 * q + 2], res[0][4 * q + 3]);
+        cv(wave)[q * 64 + lane] = make_float4(res[0][4 * q], res[0][4 * q + 1], res[0][4 * q + 2], res[0][4 * q + 3]);
     __syncthreads();
     if (wave != 0) return;
     // the trees from the lowest binary digit up (the fold runs right to
@@ -703,13 +871,13 @@ __global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const 
             for (int i = 0; i + st < n; i += 2 * st)
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    float4& a = cv[((c0 + i) * 4 + q) * 64 + lane];
-                    const float4 b = cv[((c0 + i + st) * 4 + q) * 64 + lane];
+                    float4& a = cv(c0 + i)[q * 64 + lane];
+                    const float4 b = cv(c0 + i + st)[q * 64 + lane];
                     a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
                 }
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const float4 tv = cv[(c0 * 4 + q) * 64 + lane];
+            const float4 tv = cv(c0)[q * 64 + lane];
             const float t4[4] = {tv.x, tv.y, tv.z, tv.w};
 #pragma unroll
             for (int e = 0; e < 4; e++) acc[4 * q + e] = first ? t4[e] : t4[e] + acc[4 * q + e];
@@ -741,6 +909,11 @@ size_t q4k_gemm_workspace_bytes(int batch, int in_feat) {
 }
 
 int q4k_gemm_max_in_feat() { return 127 * 256; }
+
+// Whether a batch takes the GEMM rather than one GEMV slice per batch row.
+bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t) {
+    return batch >= 32 && in_feat > 0 && in_feat <= (size_t)q4k_gemm_max_in_feat();
+}
 
 template <int LV>
 static void launch_gemm_lv(dim3 grid, hipStream_t stream, const uint8_t* w, GemmWs ws, float* y, int R, int N, int M,
@@ -775,14 +948,15 @@ static int gemm_form(int R, int N, int M, int Mt) {
     return (long)((N + kTO - 1) / kTO) * ((M + kTB - 1) / kTB) < 256 ? 3 : 0;
 }
 
+template <bool Q6>
 static hipError_t launch_sk(hipStream_t stream, const uint8_t* w, GemmWs ws, float* y, int R, int N, int M, int Mt) {
     const unsigned NR = (unsigned)((N + 31) / 32);
     const int C = sk_piece(R, (int)NR * Mt), nw = sk_chunks(R, C);
     if (C == 0 || nw > kSkMaxWaves) return hipErrorInvalidValue;
-    const size_t lds = (size_t)nw * pw_lds_per_wave(1) + (size_t)nw * 4 * 64 * 16;
-    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(&q4k_gemm_sk_kernel), lds)) return e;
-    hipLaunchKernelGGL(q4k_gemm_sk_kernel, dim3(NR * (unsigned)Mt), dim3((unsigned)nw * 64), lds, stream, w, ws, y, R,
-                       N, M, C);
+    const size_t lds = (size_t)nw * sk_lds_per_wave(Q6, C);
+    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(&q4k_gemm_sk_kernel<Q6>), lds)) return e;
+    hipLaunchKernelGGL(q4k_gemm_sk_kernel<Q6>, dim3(NR * (unsigned)Mt), dim3((unsigned)nw * 64), lds, stream, w, ws, y,
+                       R, N, M, C);
     return hipGetLastError();
 }
 
@@ -807,11 +981,11 @@ hipError_t launch_q4k_gemm(const float* x, const uint8_t* w, float* y, int batch
         const int form = gemm_form(R, out_feat, M, Mp / 32);
         const bool pw = form != 0;
         hipLaunchKernelGGL(act_quant_tiles_kernel, dim3((unsigned)R, (unsigned)(Mp / kQuantWaves)),
-                           dim3(kQuantWaves * 64), 0, stream, x + (size_t)b0 * in_feat, ws, R, M, pw ? 1 : 0);
+                           dim3(kQuantWaves * 64), 0, stream, x + (size_t)b0 * in_feat, ws, R, M, pw ? kMinF16 : kMinI8);
         if (hipError_t e = hipGetLastError()) return e;
         float* yb = y + (size_t)b0 * out_feat;
         if (pw) {
-            const hipError_t e = form == 3 ? launch_sk(stream, w, ws, yb, R, out_feat, M, Mp / 32)
+            const hipError_t e = form == 3 ? launch_sk<false>(stream, w, ws, yb, R, out_feat, M, Mp / 32)
                                            : launch_pw(stream, w, ws, yb, R, out_feat, M, Mp / 32);
             if (e) return e;
             continue;
@@ -828,6 +1002,45 @@ hipError_t launch_q4k_gemm(const float* x, const uint8_t* w, float* y, int batch
         default: launch_gemm_lv<7>(grid, stream, w, ws, yb, R, out_feat, M, NR, TT); break;
         }
         if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
+}
+
+// Q6_K: the split-K kernel for every grid, in token chunks that fit the
+// workspace.  us, one GEMV slice per batch row against this: 11008 -> 4096 at
+// 200 tokens 1607 / 93.7, 4096 -> 14336 at 512 3231 / 202, 2048 -> 32000 at 128
+// 882 / 77, 4096 x 4096 at 16 64.7 / 13.0.  Bound by the vector work of
+// forming the operands (a 32 x 32 tile at a time): 557 instructions against 16
+// MFMAs a super-block.
+size_t q6k_gemm_token_bytes(int in_feat) { return (size_t)(in_feat / 256) * 260; }
+
+// Whether a batch takes this kernel rather than one GEMV slice per batch row:
+// from 8 rows on, from 3 where the matrix has at least 2^23 weights (us, GEMV
+// against GEMM: 4096 x 4096 at 2 rows 11.0 / 12.8, at 3 14.6 / 12.7; 11008 ->
+// 4096 at 2 rows 19.1 / 22.7, at 4 35.3 / 22.7; 1024 -> 2000 at 4 rows 10.0 /
+// 11.2; 512 -> 300 at 8 rows 13.2 / 11.3).  32-bit offsets address the weights;
+// the 11 waves that rows of 127 super-blocks need do not fit in LDS.
+constexpr int kQ6MaxR = 126;
+bool q6k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat) {
+    return in_feat > 0 && in_feat <= (size_t)kQ6MaxR * 256 && out_feat * (in_feat / 256) < ((size_t)1 << 31) / 210 &&
+           (batch >= 8 || (batch >= 3 && in_feat * out_feat >= ((size_t)1 << 23)));
+}
+
+hipError_t launch_q6k_gemm(const float* x, const uint8_t* w, float* y, int batch, int in_feat, int out_feat,
+                           void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    const int R = in_feat / 256;
+    if (R < 1 || R > kQ6MaxR || (size_t)out_feat * R >= ((size_t)1 << 31) / 210)
+        return hipErrorInvalidValue;
+    const size_t fit = (workspace_bytes - 512) / q6k_gemm_token_bytes(in_feat) / 32 * 32;
+    if (fit < 32) return hipErrorInvalidValue;
+    const int chunk = (int)(fit < (size_t)kChunkM ? fit : (size_t)kChunkM);
+    for (int b0 = 0; b0 < batch; b0 += chunk) {
+        const int M = min(batch - b0, chunk), Mp = (M + 31) / 32 * 32;
+        const GemmWs ws = gemm_ws(workspace, Mp, R);
+        hipLaunchKernelGGL(act_quant_tiles_kernel, dim3((unsigned)R, (unsigned)(Mp / kQuantWaves)),
+                           dim3(kQuantWaves * 64), 0, stream, x + (size_t)b0 * in_feat, ws, R, M, kMinNone);
+        if (hipError_t e = hipGetLastError()) return e;
+        if (hipError_t e = launch_sk<true>(stream, w, ws, y + (size_t)b0 * out_feat, R, out_feat, M, Mp / 32)) return e;
     }
     return hipSuccess;
 }

@@ -37,12 +37,25 @@ struct CachedWeight {
 constexpr size_t kScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
+// Workspace of the GEMMs (quantized activations): one slot per stream, made
+// with the context and given back with it, so that a call neither allocates
+// (it may be captured) nor shares its workspace with one on another stream.
+// A fifth stream takes over the slot used longest ago.  8 MiB holds 1795
+// tokens at 4096 inputs, 224 at 32512; Q6_K walks longer batches in chunks,
+// Q4_K takes the context's grown workspace for them.
+constexpr int kSlots = 4;
+constexpr size_t kSlotBytes = (size_t)8 << 20;
+
 struct vtq_ctx {
     int device = 0;
     int num_cus = 0;
     hipStream_t stream = nullptr;
     DevBuf dx, dy;          // device staging for the host-pointer path
-    DevBuf ws;              // kernel workspace (quantized activations of the GEMM path)
+    DevBuf ws;              // GEMM workspace of batches past a slot, grown on demand
+    void* slots = nullptr;  // kSlots x kSlotBytes
+    hipStream_t slot_stream[kSlots] = {};
+    uint64_t slot_used[kSlots] = {};  // 0: free, else the call that used it last
+    uint64_t calls = 0;
     void* scratch_ptr = nullptr;  // this device's `scratch` (vtq_linear_device_noalloc)
     void* hx = nullptr;     // pinned staging
     size_t hx_cap = 0;
@@ -91,9 +104,23 @@ int grow_host(vtq_ctx* c, void*& p, size_t& cap, size_t bytes) {
     return VTQ_OK;
 }
 
+void* stream_slot(vtq_ctx* c, hipStream_t s) {
+    int k = -1;
+    for (int i = 0; i < kSlots && k < 0; i++)
+        if (c->slot_used[i] && c->slot_stream[i] == s) k = i;
+    if (k < 0) {
+        k = 0;
+        for (int i = 1; i < kSlots; i++)
+            if (c->slot_used[i] < c->slot_used[k]) k = i;
+        c->slot_stream[k] = s;
+    }
+    c->slot_used[k] = ++c->calls;
+    return static_cast<unsigned char*>(c->slots) + (size_t)k * kSlotBytes;
+}
+
 // Shape of one dtype arm after validation.
 struct Plan {
-    enum Kind { kQ4KInt, kQ4KGemm, kQ6KInt, kCanon } kind = kCanon;
+    enum Kind { kQ4KInt, kQ4KGemm, kQ6KInt, kQ6KGemm, kCanon } kind = kCanon;
     vtq::CanonFormat fmt = vtq::kCanonQ8_0;
     size_t row_bytes = 0;
     size_t w_need = 0;  // bytes of w the kernels read
@@ -126,9 +153,7 @@ int plan_linear(vtq_ctx* c, int type, int regime, size_t w_len, size_t batch, si
             if (!mul_ok(out_feat, p->row_bytes, &need) || w_len < need)
                 return set_err(c, VTQ_E_INTERNAL, serial_names ? "linear_q4_k_integer: weight shape mismatch"
                                                                : "linear_q4_k_integer_parallel: weight shape");
-            p->kind = (batch >= (size_t)vtq::kGemmMinBatch && in_feat <= (size_t)vtq::q4k_gemm_max_in_feat())
-                          ? Plan::kQ4KGemm
-                          : Plan::kQ4KInt;
+            p->kind = vtq::q4k_gemm_faster(batch, in_feat, out_feat) ? Plan::kQ4KGemm : Plan::kQ4KInt;
         } else {
             return set_err(c, VTQ_E_INVALID_ARGUMENT, "vtq: unknown regime");
         }
@@ -141,7 +166,7 @@ int plan_linear(vtq_ctx* c, int type, int regime, size_t w_len, size_t batch, si
         if (!mul_ok(out_feat, p->row_bytes, &need) || w_len < need)
             return set_err(c, VTQ_E_INTERNAL, serial_names ? "linear_q6_k_integer: weight shape mismatch"
                                                            : "linear_q6_k_integer_parallel: weight shape");
-        p->kind = Plan::kQ6KInt;
+        p->kind = vtq::q6k_gemm_faster(batch, in_feat, out_feat) ? Plan::kQ6KGemm : Plan::kQ6KInt;
         break;
     case VTQ_TYPE_Q8_0:
     case VTQ_TYPE_Q5_0: {
@@ -269,13 +294,20 @@ int run_plan(vtq_ctx* c, const Plan& p, const float* dx, const uint8_t* dw, floa
                                                          fixed_ws_bytes);
     if (p.kind == Plan::kQ4KGemm) {
         // the launcher walks the batch in chunks that fit the workspace
+        const size_t need = vtq::q4k_gemm_workspace_bytes((int)batch, (int)in_feat);
         void* ws = fixed_ws;
+        if (!ws && need <= kSlotBytes) ws = stream_slot(c, s);
         if (!ws) {
-            int rc = grow_dev(c, c->ws, vtq::q4k_gemm_workspace_bytes((int)batch, (int)in_feat));
-            if (rc) return rc;
+            if (int rc = grow_dev(c, c->ws, need)) return rc;
             ws = c->ws.ptr;
         }
         e = vtq::launch_q4k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws, s);
+        return e == hipSuccess ? VTQ_OK : hip_fail(c, e, "kernel launch");
+    }
+    if (p.kind == Plan::kQ6KGemm) {
+        void* ws = fixed_ws ? fixed_ws : stream_slot(c, s);
+        e = vtq::launch_q6k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws,
+                                 fixed_ws ? fixed_ws_bytes : kSlotBytes, s);
         return e == hipSuccess ? VTQ_OK : hip_fail(c, e, "kernel launch");
     }
     const size_t kMaxGridY = 65535;
@@ -288,6 +320,7 @@ int run_plan(vtq_ctx* c, const Plan& p, const float* dx, const uint8_t* dw, floa
             e = vtq::launch_q4k_gemv(xb, dw, yb, nb, (int)in_feat, (int)out_feat, c->num_cus, s);
             break;
         case Plan::kQ4KGemm:
+        case Plan::kQ6KGemm:
             break;
         case Plan::kQ6KInt:
             e = vtq::launch_q6k_gemv(xb, dw, yb, nb, (int)in_feat, (int)out_feat, c->num_cus, s);
@@ -428,6 +461,11 @@ int vtq_create(int device, vtq_ctx** out) {
         delete c;
         return VTQ_E_GPU;
     }
+    if (hipMalloc(&c->slots, kSlots * kSlotBytes) != hipSuccess) {
+        (void)hipStreamDestroy(c->stream);
+        delete c;
+        return VTQ_E_GPU;
+    }
     *out = c;
     return VTQ_OK;
 }
@@ -440,6 +478,7 @@ void vtq_destroy(vtq_ctx* c) {
     if (c->dx.ptr) (void)hipFree(c->dx.ptr);
     if (c->dy.ptr) (void)hipFree(c->dy.ptr);
     if (c->ws.ptr) (void)hipFree(c->ws.ptr);
+    if (c->slots) (void)hipFree(c->slots);
     if (c->hx) (void)hipHostFree(c->hx);
     if (c->hy) (void)hipHostFree(c->hy);
     if (c->stream) (void)hipStreamDestroy(c->stream);

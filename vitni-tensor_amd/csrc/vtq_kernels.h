@@ -78,12 +78,19 @@ hipError_t launch_segment_tree(const float* part, size_t n, int nseg, float* y, 
 // attribute is set once per (device, kernel) and size, not per launch.
 hipError_t allow_dynamic_lds(const void* kernel, size_t bytes);
 
-// Prefill GEMM (batch >= kGemmMinBatch): activation pre-pass into `workspace`
-// (q4k_gemm_workspace_bytes) followed by the i8-MFMA kernel.
-constexpr int kGemmMinBatch = 32;
+// Batch GEMM: activation pre-pass into `workspace` (q4k_gemm_workspace_bytes)
+// followed by the i8-MFMA kernel, where q4k_gemm_faster says so.
+bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat);
 size_t q4k_gemm_workspace_bytes(int batch, int in_feat);
 int q4k_gemm_max_in_feat();
 hipError_t launch_q4k_gemm(const float* x, const uint8_t* w, float* y, int batch, int in_feat, int out_feat,
                            void* workspace, hipStream_t stream);
+
+// The same for Q6_K; walks the batch in chunks that fit workspace_bytes (at
+// least 32 tokens: 32 * q6k_gemm_token_bytes + 512).
+bool q6k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat);
+size_t q6k_gemm_token_bytes(int in_feat);
+hipError_t launch_q6k_gemm(const float* x, const uint8_t* w, float* y, int batch, int in_feat, int out_feat,
+                           void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 }  // namespace vtq
