@@ -910,9 +910,19 @@ size_t q4k_gemm_workspace_bytes(int batch, int in_feat) {
 
 int q4k_gemm_max_in_feat() { return 127 * 256; }
 
-// Whether a batch takes the GEMM rather than one GEMV slice per batch row.
-bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t) {
-    return batch >= 32 && in_feat > 0 && in_feat <= (size_t)q4k_gemm_max_in_feat();
+// Whether a batch takes the GEMM rather than one GEMV slice per batch row: from
+// 32 rows on always; below, from 16 rows, from 8 with at least 2^22 weights,
+// from 4 with at least 2^27 weights times rows (us, GEMV against GEMM: 8 x
+// 4096 x 11008 24.2 / 15.5, 8 x 4096 x 4096 18.5 / 12.4, 4 x 4096 x 4096 10.9 /
+// 12.0, 4 x 11008 x 4096 27.5 / 19.0, 4 x 2048 x 32000 16.8 / 15.1, 3 x 2048 x
+// 32000 13.3 / 15.2, 8 x 2048 x 2048 11.6 / 11.8, 8 x 512 x 300 9.0 / 11.9,
+// 16 x 256 x 64 14.5 / 12.0).
+bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat) {
+    if (in_feat == 0 || in_feat > (size_t)q4k_gemm_max_in_feat()) return false;
+    if (batch >= 32) return true;
+    if (out_feat * (in_feat / 256) >= ((size_t)1 << 31) / 144) return false;  // past the small grids' kernel
+    const size_t w = in_feat * out_feat;
+    return batch >= 16 || (batch >= 8 && w >= ((size_t)1 << 22)) || (batch >= 4 && batch * w >= ((size_t)1 << 27));
 }
 
 template <int LV>
