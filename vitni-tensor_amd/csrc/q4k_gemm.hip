@@ -361,8 +361,9 @@ __global__ __launch_bounds__(256, 2) void q4k_gemm_kernel(const uint8_t* __restr
 constexpr int kPwWaves = 4;
 constexpr int kPwMaxR = 16;
 __host__ __device__ constexpr int pw_level_bytes(int NT) { return NT * 4 * 64 * 16; }  // one tree level of NT tiles
+constexpr int kQ4StageBytes = 32 * 80;
 __host__ __device__ constexpr int pw_lds_per_wave(int NT) {
-    return 2 * pw_level_bytes(NT) + 2 * 32 * 4;  // levels 2 and 3, then d and dmin of the rows
+    return 2 * pw_level_bytes(NT) + 2 * 32 * 4 + kQ4StageBytes;  // levels 2 and 3, d and dmin of the rows, weights
 }
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -466,7 +467,8 @@ __device__ __forceinline__ void fold_leaves(int Rl, float4* lv, float (&res)[NT]
 // lv: this wave's LDS tree levels 2 and 3; dd: its d / dmin slots.
 template <int NT>
 __device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const GemmWs& ws, int R, int N, int M, int o0,
-                                        int tp, int s0, int Rl, float4* lv, float* dd, float (&res)[NT][16]) {
+                                        int tp, int s0, int Rl, float4* lv, v4i* stage, float* dd,
+                                        float (&res)[NT][16]) {
     constexpr int D = 4;  // k-steps of token operands in flight
     const int lane = threadIdx.x & 63;
     const int r = lane & 31, g = lane >> 5;
@@ -486,31 +488,66 @@ __device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const Gem
         d0[t] = (T * R + s0) * 128;
     }
     const uint32_t vq = 16u * lane, vd = 4u * r;
+    // Weights.  A row's block is 9 chunks of 16 bytes: the header and the two
+    // halves of the four quarters h of 32 code bytes.  They are loaded in
+    // row-contiguous order (chunk 64k + lane of the 32 rows' list) and pass
+    // through the wave's LDS, the first five chunks of every row and then, in
+    // the same place, the last four.  Read straight into the lanes that use
+    // them, each at its own row, they took 350 of a super-block's 648 cache
+    // accesses, with the vector memory path three quarters busy (14336 x 4096
+    // at 512 tokens 99.7 -> 95.0 us, 11008 x 4096 at 8 tokens 18.5 -> 16.3 us,
+    // launch included; what is left is the vector work, 510 instructions beside
+    // 34 MFMAs a super-block of two tiles).  The first part lies 5 chunks a row (odd), the second 4 with
+    // chunk c at c ^ (row/4 % 4), so the row-per-lane reads meet in no bank.
+    const uint32_t row_bytes = (uint32_t)R * 144;
+    uint32_t va[3], vb[2];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int i = min(64 * k + lane, 159), row = i / 5;
+        va[k] = (uint32_t)min(o0 + row, N - 1) * row_bytes + (uint32_t)s0 * 144 + 16u * (uint32_t)(i - 5 * row);
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int i = 64 * k + lane, row = i >> 2;
+        vb[k] = (uint32_t)min(o0 + row, N - 1) * row_bytes + (uint32_t)s0 * 144 + 80u +
+                16u * (uint32_t)((i & 3) ^ ((row >> 2) & 3));
+    }
+    v4i wa[3], wb[2];
+    auto wload = [&](uint32_t so) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) wa[k] = bload16(rw, va[k], so);
+#pragma unroll
+        for (int k = 0; k < 2; k++) wb[k] = bload16(rw, vb[k], so);
+    };
     // lane (r, g): header of row r, and code bytes 32h + 16g .. +15 of each
     // quarter h: low nibbles are k-step 2h, high nibbles k-step 2h + 1, both
     // at k = 16g .. 16g + 15 of the step (the B operand's order)
-    const uint32_t vh = (uint32_t)min(o0 + r, N - 1) * ((uint32_t)R * 144) + (uint32_t)s0 * 144, vc = vh + 16 + 16 * g;
-
-    uint4 hdr = __builtin_bit_cast(uint4, bload16(rw, vh, 0));
-    uint4 qw[4];
-#pragma unroll
-    for (int h = 0; h < 4; h++) qw[h] = __builtin_bit_cast(uint4, bload16(rw, vc + 32 * h, 0));
+    const int swz = (r >> 2) & 3;
+    wload(0);
+    __builtin_amdgcn_sched_barrier(0);
     v4i bq[NT][D];  // token operands: ring of D k-steps
 #pragma unroll
     for (int j = 0; j < D; j++)
 #pragma unroll
         for (int t = 0; t < NT; t++) bq[t][j] = bload16(rq, vq, q0[t] + j * 1024);
-    v4i bm[NT];
-    float dx[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        bm[t] = bload16(rm, vq, m0[t]);
-        dx[t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t], 0));
-    }
 
     // one super-block: the parts of every tile into p
     auto sblock = [&](int s, float (&p)[NT][16]) __attribute__((always_inline)) {
         const int sn = min(s + 1, Rl - 1);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (k < 2 || lane < 32) stage[64 * k + lane] = wa[k];
+        // this super-block's min operands and token scales: loads complete in
+        // order, so they go before the next weights
+        v4i bm[NT];
+        float ds[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            bm[t] = bload16(rm, vq, m0[t] + (uint32_t)s * 1024);
+            ds[t] = __builtin_bit_cast(float,
+                                       __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t] + (uint32_t)s * 128, 0));
+        }
+        const uint4 hdr = __builtin_bit_cast(uint4, stage[5 * r]);
         // get_scale_min_k4 (src/ops/quant.rs:267-276) of all eight sub-blocks, a byte each
         const uint32_t Y = hdr.y, Z = hdr.z, Wd = hdr.w;
         const uint32_t SCl = Y & 0x3F3F3F3Fu, Ml = Z & 0x3F3F3F3Fu;
@@ -525,21 +562,29 @@ __device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const Gem
         const uint32_t am0 = pk_f16(Ml & 255u, (Ml >> 8) & 255u), am1 = pk_f16((Ml >> 16) & 255u, Ml >> 24);
         const uint32_t am2 = pk_f16(Mh & 255u, (Mh >> 8) & 255u), am3 = pk_f16((Mh >> 16) & 255u, Mh >> 24);
         const v8h am = __builtin_bit_cast(v8h, v4i{(int)am0, (int)am1, (int)am2, (int)am3});
-        hdr = __builtin_bit_cast(uint4, bload16(rw, vh, (uint32_t)sn * 144));
         v16i c1[NT], c0[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) c1[t] = c0[t] = v16i{};
+        uint4 qw;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int h = j >> 1, sh = 4 * (j & 1);
+            if (j == 4) {
+                // the second part over the first, which has been read (a wave's LDS accesses are in order)
+                stage[lane] = wb[0];
+                stage[64 + lane] = wb[1];
+                __builtin_amdgcn_sched_barrier(0);
+                wload((uint32_t)sn * 144);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!(j & 1)) qw = __builtin_bit_cast(uint4, j < 4 ? stage[5 * r + 1 + 2 * h + g] : stage[4 * r + ((2 * h - 4 + g) ^ swz)]);
             const uint32_t SH = j < 4 ? SHl : SHh, SL = j < 4 ? SLl : SLh;
             const us2 mh = __builtin_bit_cast(us2, rep_byte16(SH, j & 3));
             const us2 ml = __builtin_bit_cast(us2, rep_byte16(SL, j & 3));
-            const uint32_t w0 = (qw[h].x >> sh) & 0x0F0F0F0Fu, w1 = (qw[h].y >> sh) & 0x0F0F0F0Fu;
-            const uint32_t w2 = (qw[h].z >> sh) & 0x0F0F0F0Fu, w3 = (qw[h].w >> sh) & 0x0F0F0F0Fu;
+            const uint32_t w0 = (qw.x >> sh) & 0x0F0F0F0Fu, w1 = (qw.y >> sh) & 0x0F0F0F0Fu;
+            const uint32_t w2 = (qw.z >> sh) & 0x0F0F0F0Fu, w3 = (qw.w >> sh) & 0x0F0F0F0Fu;
             const v4i a1 = v4i{nib_mul(w0, mh), nib_mul(w1, mh), nib_mul(w2, mh), nib_mul(w3, mh)};
             const v4i a0 = v4i{nib_mul(w0, ml), nib_mul(w1, ml), nib_mul(w2, ml), nib_mul(w3, ml)};
-            if (j & 1) qw[h] = __builtin_bit_cast(uint4, bload16(rw, vc + 32 * h, (uint32_t)sn * 144));
 #pragma unroll
             for (int t = 0; t < NT; t++) c1[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bq[t][j % D], c1[t], 0, 0, 0);
 #pragma unroll
@@ -551,15 +596,9 @@ __device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const Gem
         }
         // min term (src/ops/quant.rs:876-883): accm = sum_j m_j * bsum_j
         v16f cm[NT];
-        float ds[NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
+        for (int t = 0; t < NT; t++)
             cm[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, __builtin_bit_cast(v8h, bm[t]), v16f{}, 0, 0, 0);
-            ds[t] = dx[t];
-            bm[t] = bload16(rm, vq, m0[t] + (uint32_t)sn * 1024);
-            dx[t] = __builtin_bit_cast(float,
-                                       __builtin_amdgcn_raw_buffer_load_b32(rd, vd, d0[t] + (uint32_t)sn * 128, 0));
-        }
         // epilogue (src/ops/quant.rs:849-898): element i of a lane is row 8*(i/4) + 4*g + i%4, token r
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -752,7 +791,8 @@ __global__ __launch_bounds__(kPwWaves * 64, 2) void q4k_gemm_pw_kernel(const uin
     const int r = lane & 31, g = lane >> 5;
     const int Mt = (M + 31) / 32;
     float res[NT][16];
-    pw_tree<NT>(W, ws, R, N, M, o0, tp, 0, R, lv, dd, res);
+    v4i* stage = reinterpret_cast<v4i*>(dd + 64);
+    pw_tree<NT>(W, ws, R, N, M, o0, tp, 0, R, lv, stage, dd, res);
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         const int T = NT * tp + t, tok = T * 32 + r;
@@ -818,8 +858,8 @@ __global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const 
                                                                            int C) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x & 63, wave = wave_id();
-    // per wave: the Q6_K weight stage, in which its chunk's value goes once
-    // the chunk is folded, or (Q4_K) a place for that value; then d of the
+    // per wave: the weight stage, in which its chunk's value goes once the
+    // chunk is folded (Q4_K's stage is the smaller of the two); then d of the
     // rows (Q4_K: and dmin); then tree level 2 for pieces of more than 4
     // leaves and level 3 for more than 8
     const int kW = sk_lds_per_wave(Q6, C);
@@ -850,7 +890,7 @@ __global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const 
     if constexpr (Q6)
         pw6_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, reinterpret_cast<v4i*>(base), dd, res);
     else
-        pw_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, dd, res);
+        pw_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, reinterpret_cast<v4i*>(base), dd, res);
 #pragma unroll
     for (int q = 0; q < 4; q++)
         cv(wave)[q * 64 + lane] = make_float4(res[0][4 * q], res[0][4 * q + 1], res[0][4 * q + 2], res[0][4 * q + 3]);
