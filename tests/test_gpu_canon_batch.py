@@ -1,4 +1,5 @@
-"""GPU parity of the batched pinned dot (canon_gemm.hip) against the oracle, bit for bit.
+"""GPU parity of the batched pinned dot (canon_gemm.hip,
+canon_gemm_split.hip) against the oracle, bit for bit.
 
 The shapes are large enough for the dispatch to prefer the batch kernel and
 cover its four forms (four, two and one wave to a tile of 16 rows x 16 tokens,
@@ -17,11 +18,13 @@ from test_gpu_parity import F, check
 
 pytestmark = pytest.mark.gpu
 
-BLOCK_SHAPES = [(150, 992, 300), (45, 512, 2011), (300, 64, 9000), (67, 160, 10001), (100, 8224, 240), (90, 16640, 270)]
-Q4K_SHAPES = [(45, 512, 2011), (40, 256, 5000), (260, 256, 9001), (33, 4352, 1030), (34, 8448, 1030)]
-F32_SHAPES = [(70, 1001, 700), (35, 100, 9003), (260, 33, 9001), (64, 32, 12000), (80, 4097, 513), (65, 8197, 259)]
+BLOCK_SHAPES = [(150, 992, 300), (45, 512, 2011), (300, 64, 9000), (67, 160, 10001), (100, 8224, 240), (90, 16640, 270),
+                (150, 1056, 1530)]
+Q4K_SHAPES = [(45, 512, 2011), (40, 256, 5000), (260, 256, 9001), (33, 4352, 1030), (34, 8448, 1030), (150, 1280, 1530)]
+F32_SHAPES = [(70, 1001, 700), (35, 100, 9003), (260, 33, 9001), (64, 32, 12000), (80, 4097, 513), (65, 8197, 259),
+              (150, 1030, 1530)]
 CASES = [(t, 0, *s) for t in (vtq.Q8_0, vtq.Q5_0, vtq.Q4_0) for s in BLOCK_SHAPES] \
-    + [(vtq.Q4_K, 1, *s) for s in Q4K_SHAPES] + [(vtq.F32, 0, *s) for s in F32_SHAPES]
+    + [(vtq.Q4_0, 0, 17, 8288, 6200)] + [(vtq.Q4_K, 1, *s) for s in Q4K_SHAPES] + [(vtq.F32, 0, *s) for s in F32_SHAPES]
 
 
 def weights(t, out_f, in_f, seed):

@@ -27,6 +27,8 @@ hipError_t launch_canon_gemv(CanonFormat fmt, const float* x, const uint8_t* w, 
 bool canon_gemm_faster(CanonFormat fmt, int batch, int in_feat, int out_feat);
 hipError_t launch_canon_gemm(CanonFormat fmt, const float* x, const uint8_t* w, size_t row_bytes, float* y, int batch,
                              int in_feat, int out_feat, hipStream_t stream);
+hipError_t launch_canon_gemm_split(CanonFormat fmt, int cs, const float* x, const uint8_t* w, size_t row_bytes, float* y,
+                                   int batch, int in_feat, int out_feat, hipStream_t stream);  // cs 2 or 4
 // Decode-step GEMV (integer regime, Q4_K = 12 / Q6_K = 14, batch 1): the
 // output rows are the concatenation of up to three matrices that share x
 // (unused slots have rows 0).  Epilogues: store, accumulate into y (the
