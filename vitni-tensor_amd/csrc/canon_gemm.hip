@@ -368,12 +368,16 @@ struct GmForm {
 };
 constexpr GmForm kGmForms[] = {{1, 4, 350, 520, 245}, {1, 2, 550, 855, 408}, {1, 1, 1000, 1600, 800},
                                {2, 1, 1780, 2950, 1475}};
+// F32 rows aren't staged, so with CS = 4 four waves gather each row, 16 loads of
+// 64 cache accesses a tile and step: the vector memory path's time on a full CU.
+// (64 tokens of 2048 x 2048: 33.2 us with CS = 4, 19.5 with CS = 2.)
+constexpr GmForm kGmF32Split4 = {1, 4, 430, 940, 470};
 
-int gm_pick(int batch, int n, int out_feat, long* ns) {
+int gm_pick(CanonFormat fmt, int batch, int n, int out_feat, long* ns) {
     int best = 0;
     *ns = 0;
     for (int f = 0; f < 4; f++) {
-        const GmForm& k = kGmForms[f];
+        const GmForm& k = f == 0 && fmt == kCanonF32 ? kGmF32Split4 : kGmForms[f];
         const long tiles = (long)((out_feat + 15) / 16) * ((batch + 16 * k.nt - 1) / (16 * k.nt));
         const long waves = (tiles * k.cs + 1023) / 1024, whole = (k.cs > 1 ? 4 : 1) * kStep;
         const long steps = (n + whole - 1) / whole * (whole / kStep);
@@ -389,13 +393,13 @@ int gm_pick(int batch, int n, int out_feat, long* ns) {
 // time is its weights decoded per nanosecond (measured with the shapes above:
 // Q8_0 3600 in the LDS-resident kernel, 2000 in the windowed one; Q4_K float
 // 2300, Q4_0 2000, Q5_0 1200, F32 1000).  With those the line for Q8_0 4096 x 4096
-// lies between 4 tokens (22 us against 31) and 8 (40 against 31).
+// lies between 4 tokens (22 us against 25) and 8 (40 against 25).
 bool canon_gemm_faster(CanonFormat fmt, int batch, int in_feat, int out_feat) {
     if (batch < 2 || in_feat > canon_max_in_feat()) return false;
     const double rate = fmt == kCanonQ8_0 ? (in_feat % 256 == 0 && in_feat <= 4096 ? 3600 : 2000)
                         : fmt == kCanonQ4KFloat ? 2300 : fmt == kCanonQ4_0 ? 2000 : fmt == kCanonQ5_0 ? 1200 : 1000;
     long ns;
-    gm_pick(batch, in_feat, out_feat, &ns);
+    gm_pick(fmt, batch, in_feat, out_feat, &ns);
     return (double)batch * in_feat * out_feat / rate * 0.9 > (double)ns;
 }
 
@@ -403,7 +407,7 @@ hipError_t launch_canon_gemm(CanonFormat fmt, const float* x, const uint8_t* w, 
                              int in_feat, int out_feat, hipStream_t stream) {
     if (in_feat <= 0 || in_feat > canon_max_in_feat()) return hipErrorInvalidValue;
     long ns;
-    const GmForm& f = kGmForms[gm_pick(batch, in_feat, out_feat, &ns)];
+    const GmForm& f = kGmForms[gm_pick(fmt, batch, in_feat, out_feat, &ns)];
     if (f.cs > 1) return launch_canon_gemm_split(fmt, f.cs, x, w, row_bytes, y, batch, in_feat, out_feat, stream);
     switch (fmt) {
     case kCanonQ8_0: return launch_wide<WideQ8_0>(f.nt, x, w, row_bytes, y, batch, in_feat, out_feat, stream);
