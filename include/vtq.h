@@ -130,8 +130,9 @@ int vtq_release_weights(vtq_ctx *ctx, const uint8_t *w);
  * for the null stream) without synchronising.  d_x and d_w must be 16-byte
  * aligned, and d_w readable up to the next multiple of 16 bytes past w_len
  * (every hipMalloc or torch device allocation is: the kernels fetch whole
- * 16-byte chunks and ignore the bytes past the blob).  This is what a device-resident forward step calls; it replaces
- * the same linear_dispatch arm as vtq_linear.  Calls that overlap in time on
+ * 16-byte chunks and ignore the bytes past the blob).  This is what a
+ * device-resident forward step calls; it replaces the same linear_dispatch arm
+ * as vtq_linear.  Calls that overlap in time on
  * one context race on the context's workspace. */
 int vtq_linear_device(vtq_ctx *ctx, int ggml_type, int regime, const float *d_x,
                       const uint8_t *d_w, size_t w_len, float *d_y, size_t batch, size_t in_feat,
@@ -147,9 +148,9 @@ int vtq_linear_device(vtq_ctx *ctx, int ggml_type, int regime, const float *d_x,
  * allocated when the library loads.  Q4_K requests whose workspace would
  * exceed it (vtq::q4k_gemm_workspace_bytes: about batch x in_feat x 1.14
  * bytes, batch capped at 8192 per chunk) return VTQ_E_NOT_IMPLEMENTED with a
- * message and launch nothing; Q6_K walks the batch in chunks that fit.  Rows longer than the kernels hold (k-quant
- * beyond 32768 inputs, the canonical dot beyond 65536) keep their
- * segments' sums there too (segments x batch x out_feat x 4 bytes, plus one
+ * message and launch nothing; Q6_K walks the batch in
+ * chunks that fit.  Rows longer than the kernels hold (k-quant beyond 32768
+ * inputs, the canonical dot beyond 65536) keep their segments' sums there too (segments x batch x out_feat x 4 bytes, plus one
  * gathered segment of x per batch row for the canonical dot), with the
  * batch split into passes that fit; a single batch row that does not fit
  * is refused the same way.  All calls on one GPU share that array:

@@ -74,31 +74,59 @@ def _device_case(t, batch, in_f, out_f, seed):
 
 
 def test_batches_on_several_streams():
-    # six streams in turn over four workspace slots: the first four run
-    # without waiting for each other, the last two after them
+    # ten streams that do not wait for each other: eight have a workspace of
+    # their own, the last two take the forms without one
     import torch
 
     shapes = [(vtq.Q6_K, 40, 4096, 3000), (vtq.Q4_K, 16, 4096, 3000), (vtq.Q6_K, 64, 2048, 2000), (vtq.Q4_K, 48, 2048, 2000),
-              (vtq.Q6_K, 33, 1024, 500), (vtq.Q4_K, 20, 1024, 500)]
+              (vtq.Q6_K, 33, 1024, 500), (vtq.Q4_K, 20, 1024, 500), (vtq.Q6_K, 9, 2048, 900), (vtq.Q4_K, 33, 1024, 700),
+              (vtq.Q6_K, 20, 2048, 2000), (vtq.Q4_K, 24, 2048, 2000)]
     cases = [_device_case(*s, seed=100 + i) for i, s in enumerate(shapes)]
     with vtq.Context(0) as c:
-        streams = [torch.cuda.Stream() for _ in shapes]
+        # stream handles of this test alone, whatever torch's pool hands out twice
+        streams = {s.cuda_stream: s for s in (torch.cuda.Stream() for _ in range(64))}
+        streams = list(streams.values())[:len(shapes)]
+        assert len(streams) == len(shapes)
         torch.cuda.synchronize()
-        for group in ((0, 1, 2, 3), (4, 5)):
-            for _ in range(3):
-                for i in group:
-                    (t, b, i_f, o_f), (dx, dw, dy, _w) = shapes[i], cases[i]
-                    c.linear_device(t, 0, dx.data_ptr(), dw.data_ptr(), dw.numel(), dy.data_ptr(), b, i_f, o_f,
-                                    streams[i].cuda_stream)
-            torch.cuda.synchronize()
+        for _ in range(3):
+            for (t, b, i_f, o_f), (dx, dw, dy, _w), s in zip(shapes, cases, streams):
+                c.linear_device(t, 0, dx.data_ptr(), dw.data_ptr(), dw.numel(), dy.data_ptr(), b, i_f, o_f, s.cuda_stream)
+        torch.cuda.synchronize()
         for s, (_x, _w, dy, want) in zip(shapes, cases):
             assert_bits_equal(dy.cpu().numpy(), want, str(s))
 
 
-@pytest.mark.parametrize("t,batch,in_f,out_f", [(vtq.Q6_K, 40, 4096, 700), (vtq.Q4_K, 16, 4096, 700), (vtq.Q8_0, 64, 4096, 700)])
+def test_captured_batches_share_no_workspace():
+    # two graphs captured on one stream, replayed side by side on two others
+    import torch
+
+    shapes = [(vtq.Q6_K, 40, 4096, 3000), (vtq.Q6_K, 24, 4096, 2500)]
+    cases = [_device_case(*s, seed=400 + i) for i, s in enumerate(shapes)]
+    with vtq.Context(0) as c:
+        cap, graphs = torch.cuda.Stream(), []
+        for (t, b, i_f, o_f), (dx, dw, dy, _w) in zip(shapes, cases):
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=cap):
+                c.linear_device(t, 0, dx.data_ptr(), dw.data_ptr(), dw.numel(), dy.data_ptr(), b, i_f, o_f, cap.cuda_stream)
+        streams = [torch.cuda.Stream() for _ in graphs]
+        for _ in range(3):
+            for _x, _w, dy, _want in cases:
+                dy.fill_(float("nan"))
+            torch.cuda.synchronize()
+            for g, s in zip(graphs, streams):
+                with torch.cuda.stream(s):
+                    g.replay()
+            torch.cuda.synchronize()
+            for s, (_x, _w, dy, want) in zip(shapes, cases):
+                assert_bits_equal(dy.cpu().numpy(), want, str(s))
+        del graphs
+
+
+@pytest.mark.parametrize("t,batch,in_f,out_f", [(vtq.Q6_K, 40, 4096, 700), (vtq.Q4_K, 16, 4096, 700), (vtq.Q8_0, 64, 4096, 700),
+                                                (vtq.Q4_K, 40, 4096, 700)])
 def test_first_batch_call_under_graph_capture(t, batch, in_f, out_f):
-    # a fresh context's first call is captured (it must not allocate), then
-    # replayed with other inputs between eager calls
+    # a fresh context's first call is captured (without a workspace, or in the
+    # slot that captured calls share), then replayed with other inputs between eager calls
     import torch
 
     dx, dw, dy, want = _device_case(t, batch, in_f, out_f, seed=300)

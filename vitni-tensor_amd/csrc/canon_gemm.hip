@@ -396,6 +396,8 @@ int gm_pick(CanonFormat fmt, int batch, int n, int out_feat, long* ns) {
 // lies between 4 tokens (22 us against 25) and 8 (40 against 25).
 bool canon_gemm_faster(CanonFormat fmt, int batch, int in_feat, int out_feat) {
     if (batch < 2 || in_feat > canon_max_in_feat()) return false;
+    // a launch holds fewer than 2^32 threads; no form has more than 256 to a tile of 16 x 16
+    if ((size_t)((out_feat + 15) / 16) * ((batch + 15) / 16) >= ((size_t)1 << 24)) return false;
     const double rate = fmt == kCanonQ8_0 ? (in_feat % 256 == 0 && in_feat <= 4096 ? 3600 : 2000)
                         : fmt == kCanonQ4KFloat ? 2300 : fmt == kCanonQ4_0 ? 2000 : fmt == kCanonQ5_0 ? 1200 : 1000;
     long ns;

@@ -959,7 +959,7 @@ int q4k_gemm_max_in_feat() { return 127 * 256; }
 // 16 x 256 x 64 14.5 / 12.0).
 bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat) {
     if (in_feat == 0 || in_feat > (size_t)q4k_gemm_max_in_feat()) return false;
-    if (batch >= 32) return true;
+    if (batch >= (size_t)kGemmOnlyBatch) return true;
     if (out_feat * (in_feat / 256) >= ((size_t)1 << 31) / 144) return false;  // past the small grids' kernel
     const size_t w = in_feat * out_feat;
     return batch >= 16 || (batch >= 8 && w >= ((size_t)1 << 22)) || (batch >= 4 && batch * w >= ((size_t)1 << 27));
@@ -1083,7 +1083,9 @@ hipError_t launch_q6k_gemm(const float* x, const uint8_t* w, float* y, int batch
         return hipErrorInvalidValue;
     const size_t fit = (workspace_bytes - 512) / q6k_gemm_token_bytes(in_feat) / 32 * 32;
     if (fit < 32) return hipErrorInvalidValue;
-    const int chunk = (int)(fit < (size_t)kChunkM ? fit : (size_t)kChunkM);
+    // a launch holds fewer than 2^32 threads (that cuts a chunk of 8192 tokens past 699000 rows)
+    const size_t tiles = (((size_t)1 << 32) - 1) / ((size_t)((out_feat + 31) / 32) * kSkMaxWaves * 64);
+    const int chunk = (int)min(min(fit, (size_t)kChunkM), max(tiles, (size_t)1) * 32);
     for (int b0 = 0; b0 < batch; b0 += chunk) {
         const int M = min(batch - b0, chunk), Mp = (M + 31) / 32 * 32;
         const GemmWs ws = gemm_ws(workspace, Mp, R);

@@ -37,13 +37,16 @@ struct CachedWeight {
 constexpr size_t kScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-// Workspace of the GEMMs (quantized activations): one slot per stream, made
-// with the context and given back with it, so that a call neither allocates
-// (it may be captured) nor shares its workspace with one on another stream.
-// A fifth stream takes over the slot used longest ago.  8 MiB holds 1795
+// Workspace of the GEMMs (quantized activations): one slot per stream, made at
+// the stream's first such call and given back with the context, so that calls
+// on different streams share none.  (Made with the context they would cost
+// every context half a millisecond.)  A slot stays its stream's; calls on a
+// ninth stream, and calls under capture (a graph may be replayed on any
+// stream), take the forms that need no workspace.  A Q4_K batch that has no
+// such form then takes a slot that all such calls share.  8 MiB holds 1795
 // tokens at 4096 inputs, 224 at 32512; Q6_K walks longer batches in chunks,
 // Q4_K takes the context's grown workspace for them.
-constexpr int kSlots = 4;
+constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = (size_t)8 << 20;
 
 struct vtq_ctx {
@@ -52,10 +55,9 @@ struct vtq_ctx {
     hipStream_t stream = nullptr;
     DevBuf dx, dy;          // device staging for the host-pointer path
     DevBuf ws;              // GEMM workspace of batches past a slot, grown on demand
-    void* slots = nullptr;  // kSlots x kSlotBytes
+    void* slots[kSlots + 1] = {};  // the last one shared
     hipStream_t slot_stream[kSlots] = {};
-    uint64_t slot_used[kSlots] = {};  // 0: free, else the call that used it last
-    uint64_t calls = 0;
+    int slots_used = 0;
     void* scratch_ptr = nullptr;  // this device's `scratch` (vtq_linear_device_noalloc)
     void* hx = nullptr;     // pinned staging
     size_t hx_cap = 0;
@@ -104,18 +106,34 @@ int grow_host(vtq_ctx* c, void*& p, size_t& cap, size_t bytes) {
     return VTQ_OK;
 }
 
-void* stream_slot(vtq_ctx* c, hipStream_t s) {
-    int k = -1;
-    for (int i = 0; i < kSlots && k < 0; i++)
-        if (c->slot_used[i] && c->slot_stream[i] == s) k = i;
-    if (k < 0) {
-        k = 0;
-        for (int i = 1; i < kSlots; i++)
-            if (c->slot_used[i] < c->slot_used[k]) k = i;
-        c->slot_stream[k] = s;
+// Slot k, made on first use; null if it cannot be.
+void* slot(vtq_ctx* c, int k) {
+    if (c->slots[k]) return c->slots[k];
+    // an allocation must not break a capture, here or on another thread
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipMalloc(&c->slots[k], kSlotBytes);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        c->slots[k] = nullptr;
     }
-    c->slot_used[k] = ++c->calls;
-    return static_cast<unsigned char*>(c->slots) + (size_t)k * kSlotBytes;
+    return c->slots[k];
+}
+
+// The workspace of this stream, or null: every slot is another stream's, none
+// can be made, or the call is being captured.
+void* stream_slot(vtq_ctx* c, hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    int k = 0;
+    while (k < c->slots_used && c->slot_stream[k] != s) k++;
+    if (k == kSlots || !slot(c, k)) return nullptr;
+    if (k == c->slots_used) c->slot_stream[c->slots_used++] = s;
+    return c->slots[k];
 }
 
 // Shape of one dtype arm after validation.
@@ -292,30 +310,38 @@ int run_plan(vtq_ctx* c, const Plan& p, const float* dx, const uint8_t* dw, floa
     }
     if (segment_inputs(p, in_feat)) return run_segmented(c, p, dx, dw, dy, batch, in_feat, out_feat, s, fixed_ws,
                                                          fixed_ws_bytes);
-    if (p.kind == Plan::kQ4KGemm) {
+    Plan::Kind kind = p.kind;
+    if (kind == Plan::kQ4KGemm) {
         // the launcher walks the batch in chunks that fit the workspace
         const size_t need = vtq::q4k_gemm_workspace_bytes((int)batch, (int)in_feat);
         void* ws = fixed_ws;
         if (!ws && need <= kSlotBytes) ws = stream_slot(c, s);
-        if (!ws) {
-            if (int rc = grow_dev(c, c->ws, need)) return rc;
-            ws = c->ws.ptr;
+        if (!ws && batch < (size_t)vtq::kGemmOnlyBatch) {
+            kind = Plan::kQ4KInt;
+        } else {
+            if (!ws && need <= kSlotBytes) ws = slot(c, kSlots);
+            if (!ws) {
+                if (int rc = grow_dev(c, c->ws, need)) return rc;
+                ws = c->ws.ptr;
+            }
+            e = vtq::launch_q4k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws, s);
+            return e == hipSuccess ? VTQ_OK : hip_fail(c, e, "kernel launch");
         }
-        e = vtq::launch_q4k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws, s);
-        return e == hipSuccess ? VTQ_OK : hip_fail(c, e, "kernel launch");
     }
-    if (p.kind == Plan::kQ6KGemm) {
-        void* ws = fixed_ws ? fixed_ws : stream_slot(c, s);
-        e = vtq::launch_q6k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws,
-                                 fixed_ws ? fixed_ws_bytes : kSlotBytes, s);
-        return e == hipSuccess ? VTQ_OK : hip_fail(c, e, "kernel launch");
+    if (kind == Plan::kQ6KGemm) {
+        if (void* ws = fixed_ws ? fixed_ws : stream_slot(c, s)) {
+            e = vtq::launch_q6k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws,
+                                     fixed_ws ? fixed_ws_bytes : kSlotBytes, s);
+            return e == hipSuccess ? VTQ_OK : hip_fail(c, e, "kernel launch");
+        }
+        kind = Plan::kQ6KInt;
     }
     const size_t kMaxGridY = 65535;
     for (size_t b0 = 0; b0 < batch; b0 += kMaxGridY) {
         const int nb = (int)(batch - b0 < kMaxGridY ? batch - b0 : kMaxGridY);
         const float* xb = dx + b0 * in_feat;
         float* yb = dy + b0 * out_feat;
-        switch (p.kind) {
+        switch (kind) {
         case Plan::kQ4KInt:
             e = vtq::launch_q4k_gemv(xb, dw, yb, nb, (int)in_feat, (int)out_feat, c->num_cus, s);
             break;
@@ -461,11 +487,6 @@ int vtq_create(int device, vtq_ctx** out) {
         delete c;
         return VTQ_E_GPU;
     }
-    if (hipMalloc(&c->slots, kSlots * kSlotBytes) != hipSuccess) {
-        (void)hipStreamDestroy(c->stream);
-        delete c;
-        return VTQ_E_GPU;
-    }
     *out = c;
     return VTQ_OK;
 }
@@ -478,7 +499,8 @@ void vtq_destroy(vtq_ctx* c) {
     if (c->dx.ptr) (void)hipFree(c->dx.ptr);
     if (c->dy.ptr) (void)hipFree(c->dy.ptr);
     if (c->ws.ptr) (void)hipFree(c->ws.ptr);
-    if (c->slots) (void)hipFree(c->slots);
+    for (void* p : c->slots)
+        if (p) (void)hipFree(p);
     if (c->hx) (void)hipHostFree(c->hx);
     if (c->hy) (void)hipHostFree(c->hy);
     if (c->stream) (void)hipStreamDestroy(c->stream);

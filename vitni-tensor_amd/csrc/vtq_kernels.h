@@ -81,7 +81,10 @@ hipError_t launch_segment_tree(const float* part, size_t n, int nseg, float* y, 
 hipError_t allow_dynamic_lds(const void* kernel, size_t bytes);
 
 // Batch GEMM: activation pre-pass into `workspace` (q4k_gemm_workspace_bytes)
-// followed by the i8-MFMA kernel, where q4k_gemm_faster says so.
+// followed by the i8-MFMA kernel, where q4k_gemm_faster says so; from
+// kGemmOnlyBatch rows on in every case, as the GEMV streams the matrix once
+// per batch row (4096 x 4096: 34.3 us for 16 rows already, the GEMM 12.7).
+constexpr int kGemmOnlyBatch = 32;
 bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat);
 size_t q4k_gemm_workspace_bytes(int batch, int in_feat);
 int q4k_gemm_max_in_feat();
