@@ -24,6 +24,12 @@ Q4K_SHAPES = [(16, 256, 1), (17, 512, 33), (31, 1024, 70), (8, 4096, 1025), (4, 
               (16, 43 * 256, 100), (5, 43 * 256, 2500), (24, 127 * 256, 34), (16, 128 * 256, 9)]
 
 
+# two token tiles to a wave: one to eight waves, pieces of 4, 8 and 16 leaves, a
+# last pair of one tile, remainders of rows and tokens
+Q6K_SHAPES += [(65, 512, 12001), (96, 2048, 5700), (70, 15 * 256, 2610), (40, 4096, 5701), (33, 22 * 256, 5200),
+               (64, 43 * 256, 5130), (33, 64 * 256, 5130), (33, 72 * 256, 5121), (50, 96 * 256, 5130)]
+
+
 @pytest.mark.parametrize("batch,in_f,out_f", Q6K_SHAPES)
 def test_q6k_batch(ctx, batch, in_f, out_f):
     w = synth.weights(vtq.Q6_K, out_f, in_f, seed=in_f * 3 + out_f)

@@ -848,12 +848,28 @@ static int sk_piece(int R, int T) {
 }
 
 constexpr int kQ6StageBytes = 32 * 208;
-__host__ __device__ constexpr int sk_lds_per_wave(bool q6, int C) {
-    return (q6 ? kQ6StageBytes + 128 : 4096 + 256) + (C > 8 ? 2 : C > 4 ? 1 : 0) * pw_level_bytes(1);
+// the weight stage, or a chunk's value where that is larger
+__host__ __device__ constexpr int sk_stage_bytes(bool q6, int NT) {
+    return !q6 ? 4096 : NT * 4096 > kQ6StageBytes ? NT * 4096 : kQ6StageBytes;
+}
+__host__ __device__ constexpr int sk_lds_per_wave(bool q6, int NT, int C) {
+    return sk_stage_bytes(q6, NT) + (q6 ? 128 : 256) + (C > 8 ? 2 : C > 4 ? 1 : 0) * pw_level_bytes(NT);
 }
 
-template <bool Q6>
-__global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const uint8_t* __restrict__ W, GemmWs ws,
+// With NT = 2 (Q6_K) a wave's two token tiles need the registers of an 8-wave
+// workgroup.
+constexpr int sk_max_waves(int NT) { return NT == 2 ? 8 : kSkMaxWaves; }
+
+// The piece size with two token tiles, or 0: chunks long enough to hide a
+// wave's first loads, in as many waves and as much LDS as a workgroup has.
+static int sk_piece2(int R) {
+    for (int C = 4; C <= 16; C <<= 1)
+        if (sk_chunks(R, C) <= sk_max_waves(2) && sk_chunks(R, C) * sk_lds_per_wave(true, 2, C) <= 160 * 1024) return C;
+    return 0;
+}
+
+template <bool Q6, int NT>
+__global__ __launch_bounds__(sk_max_waves(NT) * 64, 1) void q4k_gemm_sk_kernel(const uint8_t* __restrict__ W, GemmWs ws,
                                                                            float* __restrict__ y, int R, int N, int M,
                                                                            int C) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -862,13 +878,13 @@ __global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const 
     // chunk is folded (Q4_K's stage is the smaller of the two); then d of the
     // rows (Q4_K: and dmin); then tree level 2 for pieces of more than 4
     // leaves and level 3 for more than 8
-    const int kW = sk_lds_per_wave(Q6, C);
-    constexpr int kVal = Q6 ? kQ6StageBytes : 4096, kDd = Q6 ? 128 : 256;
+    const int kW = sk_lds_per_wave(Q6, NT, C);
+    constexpr int kVal = sk_stage_bytes(Q6, NT), kDd = Q6 ? 128 : 256;
     unsigned char* const base = lds + (size_t)wave * kW;
     float* dd = reinterpret_cast<float*>(base + kVal);
     float4* lv = reinterpret_cast<float4*>(base + kVal + kDd);
-    auto cv = [&](int c) { return reinterpret_cast<float4*>(lds + (size_t)c * kW); };  // [q][lane] of chunk c
-    const int Mt = (M + 31) / 32, rt = (int)blockIdx.x / Mt, tt = (int)blockIdx.x % Mt;
+    auto cv = [&](int c) { return reinterpret_cast<float4*>(lds + (size_t)c * kW); };  // [tile][q][lane] of chunk c
+    const int Mt = (M + 31) / 32, TP = (Mt + NT - 1) / NT, rt = (int)blockIdx.x / TP, tp = (int)blockIdx.x % TP;
     const int r = lane & 31, g = lane >> 5;
     // this wave's chunk
     int s0 = 0, len = 0;
@@ -886,57 +902,64 @@ __global__ __launch_bounds__(kSkMaxWaves * 64, 1) void q4k_gemm_sk_kernel(const 
             base += size;
         }
     }
-    float res[1][16];
+    float res[NT][16];
     if constexpr (Q6)
-        pw6_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, reinterpret_cast<v4i*>(base), dd, res);
+        pw6_tree<NT>(W, ws, R, N, M, rt * 32, tp, s0, len, lv, reinterpret_cast<v4i*>(base), dd, res);
     else
-        pw_tree<1>(W, ws, R, N, M, rt * 32, tt, s0, len, lv, reinterpret_cast<v4i*>(base), dd, res);
+        pw_tree<NT>(W, ws, R, N, M, rt * 32, tp, s0, len, lv, reinterpret_cast<v4i*>(base), dd, res);
 #pragma unroll
-    for (int q = 0; q < 4; q++)
-        cv(wave)[q * 64 + lane] = make_float4(res[0][4 * q], res[0][4 * q + 1], res[0][4 * q + 2], res[0][4 * q + 3]);
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            cv(wave)[t * 256 + q * 64 + lane] =
+                make_float4(res[t][4 * q], res[t][4 * q + 1], res[t][4 * q + 2], res[t][4 * q + 3]);
     __syncthreads();
-    if (wave != 0) return;
-    // the trees from the lowest binary digit up (the fold runs right to
-    // left); a tree's first chunk follows the chunks of the digits above it
-    auto pieces = [&](int k) { return (1 << k) >= C ? (1 << k) / C : 1; };
-    float acc[16];
-    bool first = true;
-    for (int k = 0; k < 7; k++) {
-        if (!((R >> k) & 1)) continue;
-        int c0 = 0;
-        for (int k2 = k + 1; k2 < 7; k2++)
-            if ((R >> k2) & 1) c0 += pieces(k2);
-        const int n = pieces(k);
-        for (int st = 1; st < n; st <<= 1)
-            for (int i = 0; i + st < n; i += 2 * st)
+    // wave t combines the values of token tile t (a lone wave takes both in turn)
+    const int nw = NT == 1 ? 1 : (int)blockDim.x >> 6;
+    if (NT == 1 && wave) return;
+    for (int t = wave; t < NT; t += nw) {
+        // the trees from the lowest binary digit up (the fold runs right to
+        // left); a tree's first chunk follows the chunks of the digits above it
+        auto pieces = [&](int k) { return (1 << k) >= C ? (1 << k) / C : 1; };
+        float acc[16];
+        bool first = true;
+        for (int k = 0; k < 7; k++) {
+            if (!((R >> k) & 1)) continue;
+            int c0 = 0;
+            for (int k2 = k + 1; k2 < 7; k2++)
+                if ((R >> k2) & 1) c0 += pieces(k2);
+            const int n = pieces(k);
+            for (int st = 1; st < n; st <<= 1)
+                for (int i = 0; i + st < n; i += 2 * st)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    float4& a = cv(c0 + i)[q * 64 + lane];
-                    const float4 b = cv(c0 + i + st)[q * 64 + lane];
-                    a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
-                }
+                    for (int q = 0; q < 4; q++) {
+                        float4& a = cv(c0 + i)[t * 256 + q * 64 + lane];
+                        const float4 b = cv(c0 + i + st)[t * 256 + q * 64 + lane];
+                        a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+                    }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float4 tv = cv(c0)[q * 64 + lane];
-            const float t4[4] = {tv.x, tv.y, tv.z, tv.w};
+            for (int q = 0; q < 4; q++) {
+                const float4 tv = cv(c0)[t * 256 + q * 64 + lane];
+                const float t4[4] = {tv.x, tv.y, tv.z, tv.w};
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc[4 * q + e] = first ? t4[e] : t4[e] + acc[4 * q + e];
+                for (int e = 0; e < 4; e++) acc[4 * q + e] = first ? t4[e] : t4[e] + acc[4 * q + e];
+            }
+            first = false;
         }
-        first = false;
-    }
-    const int tok = tt * 32 + r;
-    if (tok < M) {
-        float* yrow = y + (size_t)tok * N;
-        const bool vec = (N & 3) == 0;
+        const int tok = (NT * tp + t) * 32 + r;
+        if (tok < M) {
+            float* yrow = y + (size_t)tok * N;
+            const bool vec = (N & 3) == 0;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int o = rt * 32 + 8 * q + 4 * g;
-            if (vec && o + 3 < N) {
-                *reinterpret_cast<float4*>(yrow + o) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-            } else {
+            for (int q = 0; q < 4; q++) {
+                const int o = rt * 32 + 8 * q + 4 * g;
+                if (vec && o + 3 < N) {
+                    *reinterpret_cast<float4*>(yrow + o) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+                } else {
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (o + e < N) yrow[o + e] = acc[4 * q + e];
+                    for (int e = 0; e < 4; e++)
+                        if (o + e < N) yrow[o + e] = acc[4 * q + e];
+                }
             }
         }
     }
@@ -998,16 +1021,36 @@ static int gemm_form(int R, int N, int M, int Mt) {
     return (long)((N + kTO - 1) / kTO) * ((M + kTB - 1) / kTB) < 256 ? 3 : 0;
 }
 
+template <bool Q6, int NT>
+static hipError_t launch_sk_t(hipStream_t stream, const uint8_t* w, GemmWs ws, float* y, int R, int N, int M, int Mt, int C) {
+    const unsigned NR = (unsigned)((N + 31) / 32), TP = (unsigned)((Mt + NT - 1) / NT);
+    const int nw = sk_chunks(R, C);
+    if (C == 0 || nw > sk_max_waves(NT)) return hipErrorInvalidValue;
+    const size_t lds = (size_t)nw * sk_lds_per_wave(Q6, NT, C);
+    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(&q4k_gemm_sk_kernel<Q6, NT>), lds)) return e;
+    hipLaunchKernelGGL((q4k_gemm_sk_kernel<Q6, NT>), dim3(NR * TP), dim3((unsigned)nw * 64), lds, stream, w, ws, y, R, N, M, C);
+    return hipGetLastError();
+}
+
 template <bool Q6>
 static hipError_t launch_sk(hipStream_t stream, const uint8_t* w, GemmWs ws, float* y, int R, int N, int M, int Mt) {
-    const unsigned NR = (unsigned)((N + 31) / 32);
-    const int C = sk_piece(R, (int)NR * Mt), nw = sk_chunks(R, C);
-    if (C == 0 || nw > kSkMaxWaves) return hipErrorInvalidValue;
-    const size_t lds = (size_t)nw * sk_lds_per_wave(Q6, C);
-    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(&q4k_gemm_sk_kernel<Q6>), lds)) return e;
-    hipLaunchKernelGGL(q4k_gemm_sk_kernel<Q6>, dim3(NR * (unsigned)Mt), dim3((unsigned)nw * 64), lds, stream, w, ws, y,
-                       R, N, M, C);
-    return hipGetLastError();
+    const int NR = (N + 31) / 32;
+    if constexpr (Q6) {
+        // Two token tiles to a wave, where the workgroups and waves then still
+        // keep most of the chip busy (us, one tile against two, in brackets
+        // workgroups x waves of the second form): 11008 -> 4096 at 200 tokens
+        // 96.7 / 68.9 [512 x 7], at 96 52.4 / 33.5 [256 x 7], at 64 27.7 / 32.2 [128 x
+        // 7]; 11008 -> 6000 at 64 52.2 / 31.8 [188 x 7]; 5632 -> 2048 at 192 27.1 /
+        // 21.3 [192 x 6], at 128 17.6 / 18.9 [128 x 6]; 4096 -> 2048 at 192 19.4 / 15.7
+        // [192 x 4]; 4096 -> 14336 at 512 197 / 129; 2048 -> 32000 at 128 75.0 / 42.6.
+        // Rows of one super-block gain at some sizes and lose at others (512
+        // tokens, 10000 rows 14.9 / 15.7).
+        const int C = sk_piece2(R);
+        const long wgs = (long)NR * ((Mt + 1) / 2);
+        if (C && R > 1 && Mt > 1 && wgs >= 160 && wgs * sk_chunks(R, C) >= 700)
+            return launch_sk_t<true, 2>(stream, w, ws, y, R, N, M, Mt, C);
+    }
+    return launch_sk_t<Q6, 1>(stream, w, ws, y, R, N, M, Mt, sk_piece(R, NR * Mt));
 }
 
 static hipError_t launch_pw(hipStream_t stream, const uint8_t* w, GemmWs ws, float* y, int R, int N, int M, int Mt) {
@@ -1058,10 +1101,11 @@ hipError_t launch_q4k_gemm(const float* x, const uint8_t* w, float* y, int batch
 
 // Q6_K: the split-K kernel for every grid, in token chunks that fit the
 // workspace.  us, one GEMV slice per batch row against this: 11008 -> 4096 at
-// 200 tokens 1607 / 93.7, 4096 -> 14336 at 512 3231 / 202, 2048 -> 32000 at 128
-// 882 / 77, 4096 x 4096 at 16 64.7 / 13.0.  Bound by the vector work of
-// forming the operands (a 32 x 32 tile at a time): 557 instructions against 16
-// MFMAs a super-block.
+// 200 tokens 1607 / 68.9, 4096 -> 14336 at 512 3231 / 129, 2048 -> 32000 at 128
+// 882 / 42.6, 4096 x 4096 at 16 64.7 / 13.0.  Bound by what a 32-row super-block
+// costs before its MFMAs, 350 vector instructions and some 600 of 727 cache
+// accesses, which is why large grids take two token tiles to a wave: the same
+// weights, loaded and split once, multiply both (sizes at launch_sk).
 size_t q6k_gemm_token_bytes(int in_feat) { return (size_t)(in_feat / 256) * 260; }
 
 // Whether a batch takes this kernel rather than one GEMV slice per batch row:
