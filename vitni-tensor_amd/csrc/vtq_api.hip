@@ -39,11 +39,12 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // Workspace of the GEMMs (quantized activations): one slot per stream, made at
 // the stream's first such call and given back with the context, so that calls
-// on different streams share none.  A slot stays its stream's; calls on a ninth stream, and calls under capture (a graph may be replayed on any
-// stream), take the forms that need no workspace.  A Q4_K batch that has no
-// such form then takes a slot that all such calls share.  8 MiB holds 1795
-// tokens at 4096 inputs, 224 at 32512; Q6_K walks longer batches in chunks,
-// Q4_K takes the context's grown workspace for them.
+// on different streams share none.  A slot stays its stream's; calls on a ninth
+// stream, and calls under capture (a graph may be replayed on any stream), take
+// the forms that need no workspace.  A Q4_K batch that has no such form then
+// takes a slot that all such calls share.  8 MiB holds 1795 tokens at 4096
+// inputs, 224 at 32512; Q6_K walks longer batches in chunks, Q4_K takes the
+// context's grown workspace for them.
 constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = (size_t)8 << 20;
 
