@@ -41,7 +41,7 @@ namespace vtq {
 namespace gm {
 
 constexpr int kChunk = 8192;
-constexpr int kStep = 64;
+constexpr int kStep = kGmStep;
 constexpr int kMaxLevels = 3;                // at most 8 chunks (in_feat <= 65536)
 constexpr int kWord3 = 0x00020000;           // raw buffer descriptor word 3, gfx9 family
 constexpr uint32_t kOutOfRange = 0x80000000u;

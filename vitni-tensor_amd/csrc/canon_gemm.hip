@@ -1,6 +1,6 @@
 // canon_gemm.hip -- the pinned 8-lane fp32 dot over a batch of activation rows
-// (see canon_gemm.h): the kernel of large grids, and the choice between the
-// batch kernels.
+// (see canon_gemm.h): the kernel of large grids, and the launcher of the batch
+// kernels (their choice: vtq_rules.h).
 //
 // A wave owns all eight chains of its 16 rows and gathers its own weights, the
 // activations pass through LDS a step at a time.
@@ -353,57 +353,7 @@ hipError_t launch_wide(int nt, const float* x, const uint8_t* w, size_t row_byte
     return hipGetLastError();
 }
 
-// The forms (CS = 1 here, CS = 2 and 4 in canon_gemm_split.hip) and the time of
-// one in nanoseconds, as measured over 21 shapes (2 to 512 tokens, 256 to 11008
-// inputs, 64 to 32000 rows): what counts is the steps of a row and how many
-// waves each of the 1024 SIMDs gets in turn.  A lone wave waits for its own
-// loads and barriers, so its step costs more than a shared SIMD's.  The split
-// forms go by whole windows of four steps.  (Q8_0 4096 x 4096, us, with CS = 1 / 2
-// / 4: 16 tokens 65 / 38 / 25; 32 tokens 65 / 38 / 35; 64 tokens 65 / 58 / 65;
-// 128 tokens 103 / 107 / 126, 115 with NT = 2; 2048 x 2048 at 512 tokens 98 with
-// NT = 1, 94 with NT = 2; 896 x 4864 at 300 tokens 65 with NT = 2, 78 with CS = 2.)
-struct GmForm {
-    int nt, cs;
-    long lone, pair, more;  // ns a step: one wave per SIMD, two, each of more
-};
-constexpr GmForm kGmForms[] = {{1, 4, 350, 520, 245}, {1, 2, 550, 855, 408}, {1, 1, 1000, 1600, 800},
-                               {2, 1, 1780, 2950, 1475}};
-// F32 rows aren't staged, so with CS = 4 four waves gather each row, 16 loads of
-// 64 cache accesses a tile and step: the vector memory path's time on a full CU.
-// (64 tokens of 2048 x 2048: 33.2 us with CS = 4, 19.5 with CS = 2.)
-constexpr GmForm kGmF32Split4 = {1, 4, 430, 940, 470};
-
-int gm_pick(CanonFormat fmt, int batch, int n, int out_feat, long* ns) {
-    int best = 0;
-    *ns = 0;
-    for (int f = 0; f < 4; f++) {
-        const GmForm& k = f == 0 && fmt == kCanonF32 ? kGmF32Split4 : kGmForms[f];
-        const long tiles = (long)((out_feat + 15) / 16) * ((batch + 16 * k.nt - 1) / (16 * k.nt));
-        const long waves = (tiles * k.cs + 1023) / 1024, whole = (k.cs > 1 ? 4 : 1) * kStep;
-        const long steps = (n + whole - 1) / whole * (whole / kStep);
-        const long t = steps * (waves == 1 ? k.lone : waves == 2 ? k.pair : k.more * waves) + 3000;
-        if (f == 0 || t < *ns) best = f, *ns = t;
-    }
-    return best;
-}
-
 }  // namespace
-
-// Whether the batch kernel is faster than one GEMV slice per batch row, whose
-// time is its weights decoded per nanosecond (measured with the shapes above:
-// Q8_0 3600 in the LDS-resident kernel, 2000 in the windowed one; Q4_K float
-// 2300, Q4_0 2000, Q5_0 1200, F32 1000).  With those the line for Q8_0 4096 x 4096
-// lies between 4 tokens (22 us against 25) and 8 (40 against 25).
-bool canon_gemm_faster(CanonFormat fmt, int batch, int in_feat, int out_feat) {
-    if (batch < 2 || in_feat > canon_max_in_feat()) return false;
-    // a launch holds fewer than 2^32 threads; no form has more than 256 to a tile of 16 x 16
-    if ((size_t)((out_feat + 15) / 16) * ((batch + 15) / 16) >= ((size_t)1 << 24)) return false;
-    const double rate = fmt == kCanonQ8_0 ? (in_feat % 256 == 0 && in_feat <= 4096 ? 3600 : 2000)
-                        : fmt == kCanonQ4KFloat ? 2300 : fmt == kCanonQ4_0 ? 2000 : fmt == kCanonQ5_0 ? 1200 : 1000;
-    long ns;
-    gm_pick(fmt, batch, in_feat, out_feat, &ns);
-    return (double)batch * in_feat * out_feat / rate * 0.9 > (double)ns;
-}
 
 hipError_t launch_canon_gemm(CanonFormat fmt, const float* x, const uint8_t* w, size_t row_bytes, float* y, int batch,
                              int in_feat, int out_feat, hipStream_t stream) {

@@ -709,7 +709,8 @@ hipError_t launch_canon_gemv(CanonFormat fmt, const float* x, const uint8_t* w, 
     return launch_per_lane(fmt, x, w, row_bytes, y, batch, in_feat, out_feat, stream);
 }
 
-int canon_max_in_feat() { return kMaxChunkSlots * kChunk; }
+static_assert(kMaxChunkSlots * kChunk == kCanonMaxInFeat, "what a wave's chunk slots hold");
+int canon_max_in_feat() { return kCanonMaxInFeat; }
 
 hipError_t launch_canon_segment(CanonFormat fmt, const float* x, const uint8_t* w, size_t row_bytes, size_t w_avail,
                                 float* y, int batch, int seg_in, int out_feat, hipStream_t stream) {

@@ -119,10 +119,6 @@ __global__ __launch_bounds__(kQuantWaves * 64) void act_quant_tiles_kernel(const
 
 // ---------------------------------------------------------------- GEMM
 
-constexpr int kTO = 32;        // weight rows per workgroup
-constexpr int kTB = 128;       // tokens per workgroup (4 waves x 32)
-constexpr int kChunkM = 8192;  // tokens per launch pair (bounds the workspace)
-
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 
 // Byte-wise product of four nibbles (each <= 15) with m <= 7: every byte
@@ -359,8 +355,6 @@ __global__ __launch_bounds__(256, 2) void q4k_gemm_kernel(const uint8_t* __restr
 // Template parameter NT: token tiles per wave (2 in q4k_gemm_pw_kernel; the
 // split-K kernel folds one tile per wave with pw_tree<1>).
 constexpr int kPwWaves = 4;
-constexpr int kPwMaxR = 16;
-__host__ __device__ constexpr int pw_level_bytes(int NT) { return NT * 4 * 64 * 16; }  // one tree level of NT tiles
 constexpr int kQ4StageBytes = 32 * 80;
 __host__ __device__ constexpr int pw_lds_per_wave(int NT) {
     return 2 * pw_level_bytes(NT) + 2 * 32 * 4 + kQ4StageBytes;  // levels 2 and 3, d and dmin of the rows, weights
@@ -824,49 +818,6 @@ __global__ __launch_bounds__(kPwWaves * 64, 2) void q4k_gemm_pw_kernel(const uin
 // each tree pairwise, level by level, and the trees folded right to left
 // (fixed_tree(p[0..R)) == T_high + (... + T_low)).  Any row length to 127
 // super-blocks: C <= 16 keeps pw_tree's counter within its four levels.
-constexpr int kSkMaxWaves = 12;
-
-__host__ __device__ inline int sk_chunks(int R, int C) {
-    int n = 0;
-    for (int k = 6; k >= 0; k--)
-        if ((R >> k) & 1) n += (1 << k) >= C ? (1 << k) / C : 1;
-    return n;
-}
-
-// The piece size for a grid of T tiles: the smallest that keeps the launch
-// within 2048 waves (8 per CU), else the smallest that needs at most
-// kSkMaxWaves chunks (every row length below 128 super-blocks has one).
-static int sk_piece(int R, int T) {
-    int first = 0;
-    for (int C = 1; C <= 16; C <<= 1) {
-        const int n = sk_chunks(R, C);
-        if (n > kSkMaxWaves) continue;
-        if (!first) first = C;
-        if ((long)T * n <= 2048) return C;
-    }
-    return first;
-}
-
-constexpr int kQ6StageBytes = 32 * 208;
-// the weight stage, or a chunk's value where that is larger
-__host__ __device__ constexpr int sk_stage_bytes(bool q6, int NT) {
-    return !q6 ? 4096 : NT * 4096 > kQ6StageBytes ? NT * 4096 : kQ6StageBytes;
-}
-__host__ __device__ constexpr int sk_lds_per_wave(bool q6, int NT, int C) {
-    return sk_stage_bytes(q6, NT) + (q6 ? 128 : 256) + (C > 8 ? 2 : C > 4 ? 1 : 0) * pw_level_bytes(NT);
-}
-
-// With NT = 2 (Q6_K) a wave's two token tiles need the registers of an 8-wave
-// workgroup.
-constexpr int sk_max_waves(int NT) { return NT == 2 ? 8 : kSkMaxWaves; }
-
-// The piece size with two token tiles, or 0: chunks long enough to hide a
-// wave's first loads, in as many waves and as much LDS as a workgroup has.
-static int sk_piece2(int R) {
-    for (int C = 4; C <= 16; C <<= 1)
-        if (sk_chunks(R, C) <= sk_max_waves(2) && sk_chunks(R, C) * sk_lds_per_wave(true, 2, C) <= 160 * 1024) return C;
-    return 0;
-}
 
 template <bool Q6, int NT>
 __global__ __launch_bounds__(sk_max_waves(NT) * 64, 1) void q4k_gemm_sk_kernel(const uint8_t* __restrict__ W, GemmWs ws,
@@ -971,23 +922,6 @@ size_t q4k_gemm_workspace_bytes(int batch, int in_feat) {
     return align256((size_t)Mp * R * 256) + align256((size_t)Mp * R * 4) + (size_t)Mp * R * 32;
 }
 
-int q4k_gemm_max_in_feat() { return 127 * 256; }
-
-// Whether a batch takes the GEMM rather than one GEMV slice per batch row: from
-// 32 rows on always; below, from 16 rows, from 8 with at least 2^22 weights,
-// from 4 with at least 2^27 weights times rows (us, GEMV against GEMM: 8 x
-// 4096 x 11008 24.2 / 15.5, 8 x 4096 x 4096 18.5 / 12.4, 4 x 4096 x 4096 10.9 /
-// 12.0, 4 x 11008 x 4096 27.5 / 19.0, 4 x 2048 x 32000 16.8 / 15.1, 3 x 2048 x
-// 32000 13.3 / 15.2, 8 x 2048 x 2048 11.6 / 11.8, 8 x 512 x 300 9.0 / 11.9,
-// 16 x 256 x 64 14.5 / 12.0).
-bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat) {
-    if (in_feat == 0 || in_feat > (size_t)q4k_gemm_max_in_feat()) return false;
-    if (batch >= (size_t)kGemmOnlyBatch) return true;
-    if (out_feat * (in_feat / 256) >= ((size_t)1 << 31) / 144) return false;  // past the small grids' kernel
-    const size_t w = in_feat * out_feat;
-    return batch >= 16 || (batch >= 8 && w >= ((size_t)1 << 22)) || (batch >= 4 && batch * w >= ((size_t)1 << 27));
-}
-
 template <int LV>
 static void launch_gemm_lv(dim3 grid, hipStream_t stream, const uint8_t* w, GemmWs ws, float* y, int R, int N, int M,
                            int NR, int TT) {
@@ -1002,23 +936,6 @@ static hipError_t launch_pw_t(hipStream_t stream, const uint8_t* w, GemmWs ws, f
     hipLaunchKernelGGL((q4k_gemm_pw_kernel<NT>), dim3((unsigned)NG * (unsigned)TP), dim3(kPwWaves * 64), lds,
                        stream, w, ws, y, R, N, M, NG, TP);
     return hipGetLastError();
-}
-
-// Which kernel takes a launch (M tokens in Mt 32-token tiles): 3 the
-// split-K kernel, for grids too small to fill the chip; else 2 the per-wave
-// kernel with two token tiles per wave for rows of at most 16 super-blocks,
-// 0 the LDS-operand kernel for longer rows.  Split-K takes rows of at most 16
-// super-blocks up to 1024 tiles of 32 x 32, and longer rows where the
-// LDS-operand kernel would launch fewer than 256 workgroups (measured
-// crossovers, pre-pass included: 4096 x 4096 at 256 tokens 25.5 against
-// 26.3 us for the LDS-operand kernel, 11264 x 2048 at 96 tokens 19.5 against
-// 18.8 us for the per-wave kernel; 4096 x 11008 at 128 tokens 43.4 against
-// 56.5 us, at 256 tokens 76.6 against 59.3 us).  The split-K and per-wave
-// forms address the weights with 32-bit buffer offsets.
-static int gemm_form(int R, int N, int M, int Mt) {
-    if ((size_t)N * R * 144 >= ((size_t)1 << 31)) return 0;
-    if (R <= kPwMaxR) return (long)((N + 31) / 32) * Mt <= 1024 ? 3 : 2;
-    return (long)((N + kTO - 1) / kTO) * ((M + kTB - 1) / kTB) < 256 ? 3 : 0;
 }
 
 template <bool Q6, int NT>
@@ -1036,19 +953,7 @@ template <bool Q6>
 static hipError_t launch_sk(hipStream_t stream, const uint8_t* w, GemmWs ws, float* y, int R, int N, int M, int Mt) {
     const int NR = (N + 31) / 32;
     if constexpr (Q6) {
-        // Two token tiles to a wave, where the workgroups and waves then still
-        // keep most of the chip busy (us, one tile against two, in brackets
-        // workgroups x waves of the second form): 11008 -> 4096 at 200 tokens
-        // 96.7 / 68.9 [512 x 7], at 96 52.4 / 33.5 [256 x 7], at 64 27.7 / 32.2 [128 x
-        // 7]; 11008 -> 6000 at 64 52.2 / 31.8 [188 x 7]; 5632 -> 2048 at 192 27.1 /
-        // 21.3 [192 x 6], at 128 17.6 / 18.9 [128 x 6]; 4096 -> 2048 at 192 19.4 / 15.7
-        // [192 x 4]; 4096 -> 14336 at 512 197 / 129; 2048 -> 32000 at 128 75.0 / 42.6.
-        // Rows of one super-block gain at some sizes and lose at others (512
-        // tokens, 10000 rows 14.9 / 15.7).
-        const int C = sk_piece2(R);
-        const long wgs = (long)NR * ((Mt + 1) / 2);
-        if (C && R > 1 && Mt > 1 && wgs >= 160 && wgs * sk_chunks(R, C) >= 700)
-            return launch_sk_t<true, 2>(stream, w, ws, y, R, N, M, Mt, C);
+        if (const int C = q6k_two_tiles(R, NR, Mt)) return launch_sk_t<true, 2>(stream, w, ws, y, R, N, M, Mt, C);
     }
     return launch_sk_t<Q6, 1>(stream, w, ws, y, R, N, M, Mt, sk_piece(R, NR * Mt));
 }
@@ -1105,20 +1010,8 @@ hipError_t launch_q4k_gemm(const float* x, const uint8_t* w, float* y, int batch
 // 882 / 42.6, 4096 x 4096 at 16 64.7 / 13.0.  Bound by what a 32-row super-block
 // costs before its MFMAs, 350 vector instructions and some 600 of 727 cache
 // accesses, which is why large grids take two token tiles to a wave: the same
-// weights, loaded and split once, multiply both (sizes at launch_sk).
+// weights, loaded and split once, multiply both (sizes at q6k_two_tiles).
 size_t q6k_gemm_token_bytes(int in_feat) { return (size_t)(in_feat / 256) * 260; }
-
-// Whether a batch takes this kernel rather than one GEMV slice per batch row:
-// from 8 rows on, from 3 where the matrix has at least 2^23 weights (us, GEMV
-// against GEMM: 4096 x 4096 at 2 rows 11.0 / 12.8, at 3 14.6 / 12.7; 11008 ->
-// 4096 at 2 rows 19.1 / 22.7, at 4 35.3 / 22.7; 1024 -> 2000 at 4 rows 10.0 /
-// 11.2; 512 -> 300 at 8 rows 13.2 / 11.3).  32-bit offsets address the weights;
-// the 11 waves that rows of 127 super-blocks need do not fit in LDS.
-constexpr int kQ6MaxR = 126;
-bool q6k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat) {
-    return in_feat > 0 && in_feat <= (size_t)kQ6MaxR * 256 && out_feat * (in_feat / 256) < ((size_t)1 << 31) / 210 &&
-           (batch >= 8 || (batch >= 3 && in_feat * out_feat >= ((size_t)1 << 23)));
-}
 
 hipError_t launch_q6k_gemm(const float* x, const uint8_t* w, float* y, int batch, int in_feat, int out_feat,
                            void* workspace, size_t workspace_bytes, hipStream_t stream) {

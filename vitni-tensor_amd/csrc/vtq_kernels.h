@@ -7,10 +7,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
-namespace vtq {
+#include "vtq_rules.h"
 
-// Canonical-dot weight formats (8-lane pinned fp32 dot, src/ops/quant.rs:482-566).
-enum CanonFormat { kCanonQ8_0 = 0, kCanonQ5_0 = 1, kCanonQ4_0 = 2, kCanonF32 = 3, kCanonQ4KFloat = 4 };
+namespace vtq {
 
 size_t act_lds_bytes(int R);
 int kquant_max_in_feat();
@@ -22,9 +21,8 @@ hipError_t launch_q6k_gemv(const float* x, const uint8_t* w, float* y, int batch
                            int num_cus, hipStream_t stream);
 hipError_t launch_canon_gemv(CanonFormat fmt, const float* x, const uint8_t* w, size_t row_bytes, float* y,
                              int batch, int in_feat, int out_feat, int num_cus, hipStream_t stream);
-// The same dot for batch rows together (canon_gemm.hip), and whether it is
-// the faster one.
-bool canon_gemm_faster(CanonFormat fmt, int batch, int in_feat, int out_feat);
+// The same dot for batch rows together (canon_gemm.hip), where
+// canon_gemm_faster says so.
 hipError_t launch_canon_gemm(CanonFormat fmt, const float* x, const uint8_t* w, size_t row_bytes, float* y, int batch,
                              int in_feat, int out_feat, hipStream_t stream);
 hipError_t launch_canon_gemm_split(CanonFormat fmt, int cs, const float* x, const uint8_t* w, size_t row_bytes, float* y,
@@ -81,19 +79,13 @@ hipError_t launch_segment_tree(const float* part, size_t n, int nseg, float* y, 
 hipError_t allow_dynamic_lds(const void* kernel, size_t bytes);
 
 // Batch GEMM: activation pre-pass into `workspace` (q4k_gemm_workspace_bytes)
-// followed by the i8-MFMA kernel, where q4k_gemm_faster says so; from
-// kGemmOnlyBatch rows on in every case, as the GEMV streams the matrix once
-// per batch row (4096 x 4096: 34.3 us for 16 rows already, the GEMM 12.7).
-constexpr int kGemmOnlyBatch = 32;
-bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat);
+// followed by the i8-MFMA kernel, where q4k_gemm_faster says so.
 size_t q4k_gemm_workspace_bytes(int batch, int in_feat);
-int q4k_gemm_max_in_feat();
 hipError_t launch_q4k_gemm(const float* x, const uint8_t* w, float* y, int batch, int in_feat, int out_feat,
                            void* workspace, hipStream_t stream);
 
 // The same for Q6_K; walks the batch in chunks that fit workspace_bytes (at
 // least 32 tokens: 32 * q6k_gemm_token_bytes + 512).
-bool q6k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat);
 size_t q6k_gemm_token_bytes(int in_feat);
 hipError_t launch_q6k_gemm(const float* x, const uint8_t* w, float* y, int batch, int in_feat, int out_feat,
                            void* workspace, size_t workspace_bytes, hipStream_t stream);

@@ -1,12 +1,16 @@
-// vtq_probe.hip -- measurement helpers for bench.py (libvtq_probe.so).
+// vtq_probe.hip -- helpers of the benchmark and the tests (libvtq_probe.so).
 //
-// Not part of the quantized-linear boundary (include/vtq.h): these kernels
+// Not part of the quantized-linear boundary (include/vtq.h).  The kernels
 // exist only to measure what the hardware gives a plain access pattern on
 // the same buffers the benchmark's GEMVs read, so that each GEMV's rate can
 // be quoted against a measured read ceiling as well as the published peak.
+// The queries name the form that the dispatch rules (vtq_rules.h) give a call,
+// so that a test can say which kernel it covers; they touch no GPU.
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+
+#include "vtq_rules.h"
 
 namespace {
 
@@ -38,6 +42,35 @@ int vtqp_stream_read(const void* p, size_t bytes, int workgroups, void* sink, vo
     hipLaunchKernelGGL(stream_read_kernel, dim3((unsigned)workgroups), dim3(256), 0, (hipStream_t)stream,
                        static_cast<const uint4*>(p), bytes / 16, static_cast<uint32_t*>(sink));
     return (int)hipGetLastError();
+}
+
+// The form a pinned-dot call takes: 0 one GEMV slice per batch row, else 10 *
+// token tiles of a wave + waves to a tile.
+int vtqp_canon_form(int fmt, int batch, int in_feat, int out_feat) {
+    if (fmt < 0 || fmt > vtq::kCanonQ4KFloat || batch <= 0 || in_feat <= 0 || out_feat <= 0) return -1;
+    const vtq::CanonFormat f = (vtq::CanonFormat)fmt;
+    if (!vtq::canon_gemm_faster(f, batch, in_feat, out_feat)) return 0;
+    long ns;
+    const vtq::GmForm& g = vtq::kGmForms[vtq::gm_pick(f, batch, in_feat, out_feat, &ns)];
+    return 10 * g.nt + g.cs;
+}
+
+// The form a k-quant call (Q4_K = 12 / Q6_K = 14, integer regime) takes: 0 one
+// GEMV slice per batch row, 1 the LDS-operand kernel, 2 the per-wave kernel,
+// 300 + piece the split-K kernel, 600 + piece the same with two token tiles to
+// a wave.
+int vtqp_kquant_form(int type, int batch, int in_feat, int out_feat) {
+    if ((type != 12 && type != 14) || batch <= 0 || in_feat <= 0 || in_feat % 256 || out_feat <= 0) return -1;
+    const int R = in_feat / 256, NR = (out_feat + 31) / 32;
+    const int M = batch < vtq::kChunkM ? batch : vtq::kChunkM, Mt = (M + 31) / 32;
+    if (type == 14) {
+        if (!vtq::q6k_gemm_faster(batch, in_feat, out_feat)) return 0;
+        if (const int C = vtq::q6k_two_tiles(R, NR, Mt)) return 600 + C;
+        return 300 + vtq::sk_piece(R, NR * Mt);
+    }
+    if (!vtq::q4k_gemm_faster(batch, in_feat, out_feat)) return 0;
+    const int form = vtq::gemm_form(R, out_feat, M, Mt);
+    return form == 3 ? 300 + vtq::sk_piece(R, NR * Mt) : form == 2 ? 2 : 1;
 }
 
 }  // extern "C"
