@@ -143,21 +143,22 @@ int vtq_linear_device(vtq_ctx *ctx, int ggml_type, int regime, const float *d_x,
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same computation, arguments and
  * errors as vtq_linear_device, but it calls no hipMalloc / hipFree: the
- * batch GEMM's workspace (the quantized activations; Q4_K in the integer
- * regime and Q6_K, batch > 2) lives in a fixed 32 MiB array on each GPU,
- * allocated when the library loads.  Q4_K requests whose workspace would
+ * workspace of the GEMM that Q4_K batches of 32 rows and more take in the
+ * integer regime (the quantized activations) lives in a fixed 32 MiB array on
+ * each GPU, allocated when the library loads.  Requests whose workspace would
  * exceed it (vtq::q4k_gemm_workspace_bytes: about batch x in_feat x 1.14
  * bytes, batch capped at 8192 per chunk) return VTQ_E_NOT_IMPLEMENTED with a
- * message and launch nothing; Q6_K walks the batch in
- * chunks that fit.  Rows longer than the kernels hold (k-quant beyond 32768
- * inputs, the canonical dot beyond 65536) keep their segments' sums there too (segments x batch x out_feat x 4 bytes, plus one
- * gathered segment of x per batch row for the canonical dot), with the
- * batch split into passes that fit; a single batch row that does not fit
- * is refused the same way.  All calls on one GPU share that array:
- * calls that overlap in time on one device (any context, any stream) race
- * on it and must be serialised by the caller.  Every byte a call reads from
- * the array is written earlier in the same call, so nothing needs clearing
- * between calls. */
+ * message and launch nothing.  Smaller Q4_K batches and Q6_K take the form
+ * without a workspace, one pass over the weights per batch row.  Rows longer
+ * than the kernels hold (k-quant beyond 32768 inputs, the canonical dot beyond
+ * 65536) keep their segments' sums in the array too (segments x batch x
+ * out_feat x 4 bytes, plus one gathered segment of x per batch row for the
+ * canonical dot), with the batch split into passes that fit; a single batch
+ * row that does not fit is refused the same way.  All calls on one GPU share
+ * that array: calls that use it and overlap in time on one device (any
+ * context, any stream) race on it and must be serialised by the caller.
+ * Every byte a call reads from the array is written earlier in the same call,
+ * so nothing needs clearing between calls. */
 int vtq_linear_device_noalloc(vtq_ctx *ctx, int ggml_type, int regime, const float *d_x,
                               const uint8_t *d_w, size_t w_len, float *d_y, size_t batch,
                               size_t in_feat, size_t out_feat, void *stream);

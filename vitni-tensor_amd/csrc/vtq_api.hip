@@ -298,7 +298,9 @@ int run_segmented(vtq_ctx* c, const Plan& p, const float* dx, const uint8_t* dw,
 
 // Enqueue the kernels of a validated plan.  `fixed_ws` (when not null) is a
 // caller-provided workspace of `fixed_ws_bytes` (the GEMM's size already
-// checked); else the context's workspace grows on demand.
+// checked) that calls on other streams and contexts use too; else the context's
+// workspace grows on demand.  A batch that a GEMV per row also takes runs there
+// unless the workspace is its stream's own, so that such calls may overlap.
 int run_plan(vtq_ctx* c, const Plan& p, const float* dx, const uint8_t* dw, float* dy, size_t batch,
              size_t in_feat, size_t out_feat, hipStream_t s, void* fixed_ws = nullptr, size_t fixed_ws_bytes = 0) {
     if (batch == 0 || out_feat == 0) return VTQ_OK;
@@ -313,11 +315,11 @@ int run_plan(vtq_ctx* c, const Plan& p, const float* dx, const uint8_t* dw, floa
     if (kind == Plan::kQ4KGemm) {
         // the launcher walks the batch in chunks that fit the workspace
         const size_t need = vtq::q4k_gemm_workspace_bytes((int)batch, (int)in_feat);
-        void* ws = fixed_ws;
-        if (!ws && need <= kSlotBytes) ws = stream_slot(c, s);
+        void* ws = !fixed_ws && need <= kSlotBytes ? stream_slot(c, s) : nullptr;
         if (!ws && batch < (size_t)vtq::kGemmOnlyBatch) {
             kind = Plan::kQ4KInt;
         } else {
+            if (!ws) ws = fixed_ws;
             if (!ws && need <= kSlotBytes) ws = slot(c, kSlots);
             if (!ws) {
                 if (int rc = grow_dev(c, c->ws, need)) return rc;
@@ -328,9 +330,8 @@ int run_plan(vtq_ctx* c, const Plan& p, const float* dx, const uint8_t* dw, floa
         }
     }
     if (kind == Plan::kQ6KGemm) {
-        if (void* ws = fixed_ws ? fixed_ws : stream_slot(c, s)) {
-            e = vtq::launch_q6k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws,
-                                     fixed_ws ? fixed_ws_bytes : kSlotBytes, s);
+        if (void* ws = fixed_ws ? nullptr : stream_slot(c, s)) {
+            e = vtq::launch_q6k_gemm(dx, dw, dy, (int)batch, (int)in_feat, (int)out_feat, ws, kSlotBytes, s);
             return e == hipSuccess ? VTQ_OK : hip_fail(c, e, "kernel launch");
         }
         kind = Plan::kQ6KInt;
