@@ -132,8 +132,14 @@ int vtq_release_weights(vtq_ctx *ctx, const uint8_t *w);
  * (every hipMalloc or torch device allocation is: the kernels fetch whole
  * 16-byte chunks and ignore the bytes past the blob).  This is what a
  * device-resident forward step calls; it replaces the same linear_dispatch arm
- * as vtq_linear.  Calls that overlap in time on
- * one context race on the context's workspace. */
+ * as vtq_linear.  Calls that overlap in time on one context race on the
+ * context's workspace.
+ * A batch GEMM (Q4_K in the integer regime and Q6_K) keeps its quantized
+ * activations in 8 MiB that the context allocates at a stream's first such
+ * call, for its first eight streams, and frees with itself.  On further streams,
+ * on hipStreamPerThread and under graph capture, Q6_K and Q4_K batches below
+ * 32 rows take the form without a workspace, which passes over the weights once
+ * per batch row; larger Q4_K batches share one workspace there. */
 int vtq_linear_device(vtq_ctx *ctx, int ggml_type, int regime, const float *d_x,
                       const uint8_t *d_w, size_t w_len, float *d_y, size_t batch, size_t in_feat,
                       size_t out_feat, void *stream);

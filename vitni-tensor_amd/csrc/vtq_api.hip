@@ -39,12 +39,16 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // Workspace of the GEMMs (quantized activations): one slot per stream, made at
 // the stream's first such call and given back with the context, so that calls
-// on different streams share none.  A slot stays its stream's; calls on a ninth
-// stream, and calls under capture (a graph may be replayed on any stream), take
-// the forms that need no workspace.  A Q4_K batch that has no such form then
-// takes a slot that all such calls share.  8 MiB holds 1795 tokens at 4096
-// inputs, 224 at 32512; Q6_K walks longer batches in chunks, Q4_K takes the
-// context's grown workspace for them.
+// on different streams share none.  A slot stays its stream's.  Calls on a ninth
+// stream, on hipStreamPerThread (one handle for another stream in every thread)
+// and under capture (a graph may be replayed on any stream) take the forms that
+// need no workspace.  A Q4_K batch that has no such form then takes a slot that
+// all such calls share.  8 MiB holds 1795 tokens at 4096 inputs, 224 at 32512;
+// Q6_K walks longer batches in chunks, Q4_K takes the context's grown workspace
+// for them, which streams share.  (A slot that changes hands would need an event
+// after each use: 0.9 us of a call's 27.4 us, two kernels, measured.  A handle that
+// the runtime gives out again names a stream that has waited for the old one's
+// work: destroying a stream with a 227 ms kernel in flight took 227 ms.)
 constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = (size_t)8 << 20;
 
@@ -121,8 +125,9 @@ void* slot(vtq_ctx* c, int k) {
 }
 
 // The workspace of this stream, or null: every slot is another stream's, none
-// can be made, or the call is being captured.
+// can be made, the handle is no stream of its own, or the call is being captured.
 void* stream_slot(vtq_ctx* c, hipStream_t s) {
+    if (s == hipStreamPerThread) return nullptr;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
