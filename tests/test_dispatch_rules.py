@@ -18,3 +18,19 @@ INT, FLOAT = vtq.REGIME_INTEGER, vtq.REGIME_FLOAT_FUSED
 ])
 def test_a_shape_of_each_form(args, form):
     assert probe.form(*args) == form
+
+
+@pytest.mark.parametrize("in_f,out_f", [(17 * 256, 8200), (5120, 60000), (8192, 128256), (11008, 16384), (14336, 8192),
+                                        (16384, 9000), (28672, 8192), (127 * 256, 20000), (43 * 256, 4096)])
+@pytest.mark.parametrize("batch", [4, 5, 8, 16, 31])
+def test_q4k_batches_below_32_on_long_rows_take_split_k(batch, in_f, out_f):
+    # never the LDS-operand kernel, a workgroup of which holds 128 tokens: slower than the GEMV at 4 and 5 rows
+    assert probe.form(vtq.Q4_K, INT, batch, in_f, out_f) >= 300
+
+
+@pytest.mark.parametrize("in_f", [2048, 3072, 4096])
+def test_four_q4k_rows_past_the_split_k_grids(in_f):
+    assert [probe.form(vtq.Q4_K, INT, 4, in_f, n) for n in (32769, 39999)] == [probe.GEMV] * 2
+    assert [probe.form(vtq.Q4_K, INT, 4, in_f, n) for n in (40000, 65536)] == [probe.PER_WAVE] * 2
+    assert probe.form(vtq.Q4_K, INT, 5, in_f, 32769) == probe.PER_WAVE
+    assert probe.form(vtq.Q4_K, INT, 4, in_f, 32768) >= 300

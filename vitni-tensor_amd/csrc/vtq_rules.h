@@ -129,11 +129,16 @@ inline int sk_piece2(int R) {
 // crossovers, pre-pass included: 4096 x 4096 at 256 tokens 25.5 against
 // 26.3 us for the LDS-operand kernel, 11264 x 2048 at 96 tokens 19.5 against
 // 18.8 us for the per-wave kernel; 4096 x 11008 at 128 tokens 43.4 against
-// 56.5 us, at 256 tokens 76.6 against 59.3 us).  The split-K and per-wave
-// forms address the weights with 32-bit buffer offsets.
+// 56.5 us, at 256 tokens 76.6 against 59.3 us).  Longer rows below 32 tokens
+// always take it: the LDS-operand kernel spends a workgroup of 128 tokens on
+// them and folds a row in series (us, GEMV per row / LDS-operand / split-K, 4
+// tokens: 14336 -> 8192 57 / 74 / 27, 4352 -> 8200 20.8 / 29.8 / 16.3, 8192 ->
+// 128256 391 / 405 / 186; at 31 tokens of 14336 -> 8192 357 / 71 / 27).  The
+// split-K and per-wave forms address the weights with 32-bit buffer offsets.
 inline int gemm_form(int R, int N, int M, int Mt) {
     if ((size_t)N * R * 144 >= ((size_t)1 << 31)) return 0;
     if (R <= kPwMaxR) return (long)((N + 31) / 32) * Mt <= 1024 ? 3 : 2;
+    if (M < 32) return 3;
     return (long)((N + kTO - 1) / kTO) * ((M + kTB - 1) / kTB) < 256 ? 3 : 0;
 }
 
@@ -149,12 +154,17 @@ constexpr int kQ4MaxR = 127;
 // 4096 x 11008 24.2 / 15.5, 8 x 4096 x 4096 18.5 / 12.4, 4 x 4096 x 4096 10.9 /
 // 12.0, 4 x 11008 x 4096 27.5 / 19.0, 4 x 2048 x 32000 16.8 / 15.1, 3 x 2048 x
 // 32000 13.3 / 15.2, 8 x 2048 x 2048 11.6 / 11.8, 8 x 512 x 300 9.0 / 11.9,
-// 16 x 256 x 64 14.5 / 12.0).
+// 16 x 256 x 64 14.5 / 12.0).  Four tokens on rows of 8 to 16 super-blocks gain
+// less: past 32768 outputs, where the per-wave kernel takes them in rounds of
+// 65536, they take it from 40000 on (4096 -> 33000 41.0 / 47.5, -> 40000 49.7 /
+// 48.8; 3072 -> 33000 30.9 / 36.0, -> 40000 38.0 / 37.7; 2048 -> 33000 18.7 / 24.2,
+// -> 40000 25.5 / 25.7).
 inline bool q4k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat) {
     if (in_feat == 0 || in_feat > (size_t)kQ4MaxR * 256) return false;
     if (batch >= (size_t)kGemmOnlyBatch) return true;
     if (out_feat * (in_feat / 256) >= ((size_t)1 << 31) / 144) return false;  // past the small grids' kernel
     const size_t w = in_feat * out_feat;
+    if (batch == 4 && in_feat >= 2048 && in_feat <= (size_t)kPwMaxR * 256 && out_feat > 32768 && out_feat < 40000) return false;
     return batch >= 16 || (batch >= 8 && w >= ((size_t)1 << 22)) || (batch >= 4 && batch * w >= ((size_t)1 << 27));
 }
 
