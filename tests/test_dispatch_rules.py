@@ -34,3 +34,20 @@ def test_four_q4k_rows_past_the_split_k_grids(in_f):
     assert [probe.form(vtq.Q4_K, INT, 4, in_f, n) for n in (40000, 65536)] == [probe.PER_WAVE] * 2
     assert probe.form(vtq.Q4_K, INT, 5, in_f, 32769) == probe.PER_WAVE
     assert probe.form(vtq.Q4_K, INT, 4, in_f, 32768) >= 300
+
+
+@pytest.mark.parametrize("batch,in_f,below,above", [(3, 1024, 8191, 8192), (3, 2048, 5119, 5120), (3, 4096, 4095, 4096),
+                                                    (3, 8192, 4095, 4096), (3, 14336, 2340, 2341), (4, 4096, 2047, 2048),
+                                                    (4, 8192, 2047, 2048), (4, 14336, 804, 805), (5, 8192, 1407, 1408),
+                                                    (5, 14336, 585, 586), (7, 8192, 1023, 1024)])
+def test_q6k_small_batches_of_long_rows(batch, in_f, below, above):
+    # the GEMV is faster below: 3 rows of 14336 -> 600 18.6 us against 25.3
+    assert probe.form(vtq.Q6_K, INT, batch, in_f, below) == probe.GEMV
+    assert probe.form(vtq.Q6_K, INT, batch, in_f, above) > probe.GEMV
+
+
+@pytest.mark.parametrize("in_f", [256, 4096, 126 * 256])
+def test_q6k_batches_of_eight_rows_take_the_gemm(in_f):
+    assert probe.form(vtq.Q6_K, INT, 2, in_f, 100000) == probe.GEMV
+    assert probe.form(vtq.Q6_K, INT, 8, in_f, 1) >= 300
+    assert probe.form(vtq.Q6_K, INT, 8, 127 * 256, 1) == probe.GEMV

@@ -183,16 +183,35 @@ inline int q6k_two_tiles(int R, int NR, int Mt) {
     return C && R > 1 && Mt > 1 && wgs >= 160 && wgs * sk_chunks(R, C) >= 700 ? C : 0;
 }
 
+// From how many weights on a Q6_K batch of 3 to 7 rows takes the GEMM: its time
+// below some 10 M weights is a row's chain of leaves (7.8 us and 0.3 us a
+// super-block), the GEMV's a pass over the matrix per batch row, so long rows of
+// small matrices stay with the GEMV.  us, GEMV against GEMM, either side of each
+// line: 3 rows 1024 -> 8193 12.7 / 9.0; 2048 -> 4097 9.1 / 9.9, -> 5793 11.0 / 10.2;
+// 4096 -> 2897 11.4 / 12.7, -> 4097 13.6 / 13.4; 8192 -> 2897 16.2 / 18.1, -> 4097
+// 19.3 / 18.8; 14336 -> 1656 24.7 / 25.7, -> 2341 26.7 / 26.4.  4 rows 4096 -> 2049
+// 12.3 / 12.4; 8192 -> 1449 15.4 / 17.8, -> 2049 17.9 / 17.9; 14336 -> 586 24.0 /
+// 25.8, -> 828 26.8 / 25.5.  5 rows 8192 -> 1025 16.2 / 17.7, -> 1449 18.7 / 17.9.
+inline size_t q6k_least_weights(size_t batch, int R) {
+    size_t m = 8;
+    if (batch == 3) m = R <= 4 ? 8 : R <= 8 ? 10 : R <= 16 ? 16 : 32;
+    if (batch == 4 && R > 16) m = R <= 32 ? 16 : 11;
+    if (batch == 5 && R > 16 && R <= 32) m = 11;
+    return m << 20;
+}
+
 // Whether a Q6_K batch takes the GEMM rather than one GEMV slice per batch row:
-// from 8 rows on, from 3 where the matrix has at least 2^23 weights (us, GEMV
-// against GEMM: 4096 x 4096 at 2 rows 11.0 / 12.8, at 3 14.6 / 12.7; 11008 ->
-// 4096 at 2 rows 19.1 / 22.7, at 4 35.3 / 22.7; 1024 -> 2000 at 4 rows 10.0 /
-// 11.2; 512 -> 300 at 8 rows 13.2 / 11.3).  32-bit offsets address the weights;
-// the 11 waves that rows of 127 super-blocks need do not fit in LDS.
+// from 8 rows on, from 3 with q6k_least_weights (us, GEMV against GEMM: 4096 x
+// 4096 at 2 rows 11.0 / 12.8; 11008 -> 4096 at 2 rows 19.1 / 22.7, at 4 35.3 /
+// 22.7; 1024 -> 2000 at 4 rows 10.0 / 11.2; 512 -> 300 at 8 rows 13.2 / 11.3).
+// 32-bit offsets address the weights; the 11 waves that rows of 127 super-blocks
+// need do not fit in LDS.
 constexpr int kQ6MaxR = 126;
 inline bool q6k_gemm_faster(size_t batch, size_t in_feat, size_t out_feat) {
-    return in_feat > 0 && in_feat <= (size_t)kQ6MaxR * 256 && out_feat * (in_feat / 256) < ((size_t)1 << 31) / 210 &&
-           (batch >= 8 || (batch >= 3 && in_feat * out_feat >= ((size_t)1 << 23)));
+    if (in_feat == 0 || in_feat > (size_t)kQ6MaxR * 256) return false;
+    const size_t R = in_feat / 256;
+    return out_feat * R < ((size_t)1 << 31) / 210 &&
+           (batch >= 8 || (batch >= 3 && in_feat * out_feat >= q6k_least_weights(batch, (int)R)));
 }
 
 }  // namespace vtq
