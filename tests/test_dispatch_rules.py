@@ -51,3 +51,17 @@ def test_q6k_batches_of_eight_rows_take_the_gemm(in_f):
     assert probe.form(vtq.Q6_K, INT, 2, in_f, 100000) == probe.GEMV
     assert probe.form(vtq.Q6_K, INT, 8, in_f, 1) >= 300
     assert probe.form(vtq.Q6_K, INT, 8, 127 * 256, 1) == probe.GEMV
+
+
+@pytest.mark.parametrize("t,in_f,out_f", [(vtq.Q4_0, 1536, 32000), (vtq.Q4_0, 3072, 16384), (vtq.Q4_0, 4096, 16384),
+                                          (vtq.Q4_0, 8192, 32000), (vtq.Q8_0, 4352, 32000), (vtq.Q8_0, 8192, 32000)])
+def test_two_rows_on_a_full_grid_stay_with_the_gemv(t, in_f, out_f):
+    # Q4_0 2 x 4096 -> 16384 47.5 us against 57.0 in the batch kernel; three rows 67.5 against 56.9
+    assert probe.form(t, INT, 2, in_f, out_f) == probe.GEMV
+    assert probe.form(t, INT, 3, in_f, out_f) > probe.GEMV
+
+
+@pytest.mark.parametrize("t,in_f,out_f", [(vtq.Q4_0, 11008, 16384), (vtq.Q8_0, 14336, 32000), (vtq.Q5_0, 4096, 14336),
+                                          (vtq.F32, 4096, 14336)])
+def test_two_rows_that_take_the_batch_kernel(t, in_f, out_f):
+    assert probe.form(t, INT, 2, in_f, out_f) > probe.GEMV

@@ -36,6 +36,7 @@ constexpr GmForm kGmForms[] = {{1, 4, 350, 520, 245}, {1, 2, 550, 855, 408}, {1,
 // 64 cache accesses a tile and step: the vector memory path's time on a full CU.
 // (64 tokens of 2048 x 2048: 33.2 us with CS = 4, 19.5 with CS = 2.)
 constexpr GmForm kGmF32Split4 = {1, 4, 430, 940, 470};
+constexpr long kGmLaunchNs = 3000;  // besides the steps
 
 inline int gm_pick(CanonFormat fmt, int batch, int n, int out_feat, long* ns) {
     int best = 0;
@@ -45,7 +46,7 @@ inline int gm_pick(CanonFormat fmt, int batch, int n, int out_feat, long* ns) {
         const long tiles = (long)((out_feat + 15) / 16) * ((batch + 16 * k.nt - 1) / (16 * k.nt));
         const long waves = (tiles * k.cs + 1023) / 1024, whole = (k.cs > 1 ? 4 : 1) * kGmStep;
         const long steps = (n + whole - 1) / whole * (whole / kGmStep);
-        const long t = steps * (waves == 1 ? k.lone : waves == 2 ? k.pair : k.more * waves) + 3000;
+        const long t = steps * (waves == 1 ? k.lone : waves == 2 ? k.pair : k.more * waves) + kGmLaunchNs;
         if (f == 0 || t < *ns) best = f, *ns = t;
     }
     return best;
@@ -55,16 +56,28 @@ inline int gm_pick(CanonFormat fmt, int batch, int n, int out_feat, long* ns) {
 // time is its weights decoded per nanosecond (measured with the shapes above:
 // Q8_0 3600 in the LDS-resident kernel, 2000 in the windowed one; Q4_K float
 // 2300, Q4_0 2000, Q5_0 1200, F32 1000).  With those the line for Q8_0 4096 x 4096
-// lies between 4 tokens (22 us against 25) and 8 (40 against 25).
+// lies between 4 tokens (22 us against 25) and 8 (40 against 25).  The windowed
+// kernel is faster on a grid that fills the chip, rows of one chunk that are long
+// enough to hide their start: Q4_0 2500 (2 tokens, us, GEMV against the batch
+// kernel: 4096 -> 16384 47.5 / 57.0, -> 32000 88.4 / 105.2; 1024 -> 32000 30.0 /
+// 29.7; 11008 -> 16384 190 / 148), on a smaller one 2100 (7 tokens, 3840 -> 1985 22.6 /
+// 24.4; 3, 2048 -> 8192 20.8 / 19.6), Q8_0 2900 and 2200 (8192 -> 32000 162 / 200;
+// 14336 -> 32000 447 / 348; 3 tokens, 7040 -> 15341 103 / 95, 6272 -> 6629 44.2 /
+// 50.5, 4352 -> 8192 36.0 / 35.1).
 inline bool canon_gemm_faster(CanonFormat fmt, int batch, int in_feat, int out_feat) {
     if (batch < 2 || in_feat > kCanonMaxInFeat) return false;
     // a launch holds fewer than 2^32 threads; no form has more than 256 to a tile of 16 x 16
     if ((size_t)((out_feat + 15) / 16) * ((batch + 15) / 16) >= ((size_t)1 << 24)) return false;
-    const double rate = fmt == kCanonQ8_0 ? (in_feat % 256 == 0 && in_feat <= 4096 ? 3600 : 2000)
-                        : fmt == kCanonQ4KFloat ? 2300 : fmt == kCanonQ4_0 ? 2000 : fmt == kCanonQ5_0 ? 1200 : 1000;
+    const bool one = in_feat > 1024 && in_feat <= 8192, full = one && (size_t)batch * out_feat >= 32000;
+    const double rate = fmt == kCanonQ8_0 ? (in_feat % 256 == 0 && in_feat <= 4096 ? 3600 : full ? 2900 : one ? 2200 : 2000)
+                        : fmt == kCanonQ4KFloat ? 2300
+                        : fmt == kCanonQ4_0 ? (full ? 2500 : one ? 2100 : 2000)
+                        : fmt == kCanonQ5_0 ? 1200 : 1000;
+    const double gemv = (double)batch * in_feat * out_feat / rate * 0.9;
+    if (gemv <= kGmLaunchNs) return false;
     long ns;
     gm_pick(fmt, batch, in_feat, out_feat, &ns);
-    return (double)batch * in_feat * out_feat / rate * 0.9 > (double)ns;
+    return gemv > (double)ns;
 }
 
 // ------------------------------------------------------- k-quant batch GEMM
