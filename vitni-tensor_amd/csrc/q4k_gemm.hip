@@ -120,6 +120,7 @@ __global__ __launch_bounds__(kQuantWaves * 64) void act_quant_tiles_kernel(const
 // ---------------------------------------------------------------- GEMM
 
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // y promises no more than 4 bytes
 
 // Byte-wise product of four nibbles (each <= 15) with m <= 7: every byte
 // stays below 256, so one packed 16-bit multiply carries nothing across bytes.
@@ -311,8 +312,8 @@ __global__ __launch_bounds__(256, 2) void q4k_gemm_kernel(const uint8_t* __restr
         for (int q = 0; q < 4; q++) {
             const int o = o0 + 8 * q + 4 * g;
             if (vec && o + 3 < N) {
-                *reinterpret_cast<float4*>(yrow + o) =
-                    make_float4(r16[4 * q], r16[4 * q + 1], r16[4 * q + 2], r16[4 * q + 3]);
+                *reinterpret_cast<f32x4_a4*>(yrow + o) =
+                    f32x4_a4{r16[4 * q], r16[4 * q + 1], r16[4 * q + 2], r16[4 * q + 3]};
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++)
@@ -797,8 +798,8 @@ __global__ __launch_bounds__(kPwWaves * 64, 2) void q4k_gemm_pw_kernel(const uin
             for (int q = 0; q < 4; q++) {
                 const int o = o0 + 8 * q + 4 * g;
                 if (vec && o + 3 < N) {
-                    *reinterpret_cast<float4*>(yrow + o) =
-                        make_float4(res[t][4 * q], res[t][4 * q + 1], res[t][4 * q + 2], res[t][4 * q + 3]);
+                    *reinterpret_cast<f32x4_a4*>(yrow + o) =
+                        f32x4_a4{res[t][4 * q], res[t][4 * q + 1], res[t][4 * q + 2], res[t][4 * q + 3]};
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
@@ -905,7 +906,7 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64, 1) void q4k_gemm_sk_kernel(c
             for (int q = 0; q < 4; q++) {
                 const int o = rt * 32 + 8 * q + 4 * g;
                 if (vec && o + 3 < N) {
-                    *reinterpret_cast<float4*>(yrow + o) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+                    *reinterpret_cast<f32x4_a4*>(yrow + o) = f32x4_a4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
