@@ -1,5 +1,6 @@
-"""GPU parity of every form of the batch kernels, bit for bit against the oracle.
-Each case names the form that the dispatch gives it (vtq.probe.form).
+"""GPU parity of the k-quant batch kernels where the dispatch changes form, and of
+all of them with y aligned to 4 bytes; bit for bit against the oracle.  Each case
+names the form that the dispatch gives it (vtq.probe.form).
 """
 import pytest
 
@@ -14,10 +15,12 @@ pytestmark = pytest.mark.gpu
 INT = vtq.REGIME_INTEGER
 
 
-# Q4_K batches below 32 rows on grids past those of short rows and small matrices
+# Q4_K batches below 32 rows on grids past those of short rows and small matrices,
+# and the larger pieces of long rows
 @pytest.mark.parametrize("batch,in_f,out_f,form", [(5, 17 * 256, 8200, 304), (31, 17 * 256, 8161, 304), (4, 127 * 256, 8165, 316),
                                                    (8, 256, 33000, probe.PER_WAVE), (20, 768, 32801, probe.PER_WAVE),
-                                                   (4, 2048, 33000, probe.GEMV)])
+                                                   (4, 2048, 33000, probe.GEMV), (16, 64 * 256, 40, 308),
+                                                   (16, 126 * 256, 40, 316)])
 def test_q4k_small_batches_on_large_matrices(ctx, batch, in_f, out_f, form):
     assert probe.form(vtq.Q4_K, INT, batch, in_f, out_f) == form
     w = synth.weights(vtq.Q4_K, out_f, in_f, seed=in_f + out_f)

@@ -1,11 +1,11 @@
 """GPU parity of the batched pinned dot (canon_gemm.hip,
 canon_gemm_split.hip) against the oracle, bit for bit.
 
-The shapes are large enough for the dispatch to prefer the batch kernel and
-cover its four forms (four, two and one wave to a tile of 16 rows x 16 tokens,
-one wave to 16 x 32), token and row counts either side of the tiles, rows that
-end in the middle of a 64-input step, and rows of two and three 8192-input
-chunks.
+The shapes are large enough for the dispatch to prefer a batch kernel, most of
+them its form for small grids (four waves to a tile of 16 rows x 16 tokens), and
+have token and row counts either side of the tiles, rows that end in the middle
+of a 64-input step, and rows of two and three 8192-input chunks.
+test_gpu_canon_forms.py takes every form and format through such rows by name.
 """
 import numpy as np
 import pytest
