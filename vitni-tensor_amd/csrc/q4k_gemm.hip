@@ -24,8 +24,9 @@
 //
 // Three kernels share the activation pre-pass, which writes the token codes
 // in the MFMA operand order (gemm_form picks one per launch):
-//  * q4k_gemm_pw_kernel (rows of at most 16 super-blocks): each wave forms
-//    its own weight operands in registers, no barriers;
+//  * q4k_gemm_pw_kernel (rows of at most 16 super-blocks): each wave loads its
+//    weights through its own part of LDS and forms its operands in registers,
+//    no barriers;
 //  * q4k_gemm_sk_kernel (grids too small to fill the chip): the same
 //    per-wave fold over whole fixed_tree subtrees of a row, one per wave of
 //    a workgroup, combined in the tree's order;
@@ -326,12 +327,12 @@ __global__ __launch_bounds__(256, 2) void q4k_gemm_kernel(const uint8_t* __restr
 // ------------------------------------------- per-wave operand formation
 
 // Rows of at most 16 super-blocks (in_feat <= 4096).  Each wave owns 32
-// weight rows x 64 tokens (two 32-token tiles; one tile where two would
-// leave the CUs idle) and forms the split weight
-// operands of its rows in registers, straight from the 144-byte blocks: no
-// LDS operand buffers and no workgroup barrier, so the two waves sharing a
-// SIMD drift out of phase and one's MFMAs run beside the other's epilogue.
-// One formed operand feeds the MFMAs of both tiles.
+// weight rows x 64 tokens (two 32-token tiles) and forms the split weight
+// operands of its rows in registers from the 144-byte blocks, which pass
+// through its own part of LDS (pw_tree): no shared operand buffers and no
+// workgroup barrier, so the two waves sharing a SIMD drift out of phase and
+// one's MFMAs run beside the other's epilogue.  One formed operand feeds the
+// MFMAs of both tiles.
 //
 // A workgroup is four waves on four consecutive 32-row tiles and the same 64
 // tokens, so the token operands of a super-block are fetched from L2 once per
@@ -491,9 +492,10 @@ __device__ __forceinline__ void pw_tree(const uint8_t* __restrict__ W, const Gem
     // them, each at its own row, they took 350 of a super-block's 648 cache
     // accesses, with the vector memory path three quarters busy (14336 x 4096
     // at 512 tokens 99.7 -> 95.0 us, 11008 x 4096 at 8 tokens 18.5 -> 16.3 us,
-    // launch included; what is left is the vector work, 510 instructions beside
-    // 34 MFMAs a super-block of two tiles).  The first part lies 5 chunks a row (odd), the second 4 with
-    // chunk c at c ^ (row/4 % 4), so the row-per-lane reads meet in no bank.
+    // launch included; 456 accesses are left, and 459 vector instructions beside
+    // 34 MFMAs a super-block of two tiles).  The first part lies 5 chunks a row
+    // (odd), the second 4 with chunk c at c ^ (row/4 % 4), to spread the
+    // row-per-lane reads over the banks (15% of the LDS cycles are conflicts).
     const uint32_t row_bytes = (uint32_t)R * 144;
     uint32_t va[3], vb[2];
 #pragma unroll
@@ -649,9 +651,10 @@ __device__ __forceinline__ void pw6_tree(const uint8_t* __restrict__ W, const Ge
     // of every row it touches, and the wave's LDS holds the rows 208 bytes
     // apart (13 chunks, odd: the row-per-lane reads below meet in no bank).
     // Read straight into the lanes that use them, each at its own row, they
-    // cost 2022 cache accesses a super-block instead of 727 and the 200-token
-    // case above 135 us.  (Aligned chunks, moved into place by unaligned LDS
-    // writes, cost 306 accesses but 106.7 us: such writes are slow.)
+    // cost 2022 cache accesses a super-block instead of 727, and 200 tokens of
+    // 11008 -> 4096 135 us instead of 92 (one token tile to a wave).  (Aligned
+    // chunks, moved into place by unaligned LDS writes, cost 306 accesses but
+    // 106.7 us: such writes are slow.)
     constexpr int kCh = 13, kLoads = 7;
     const uint32_t row_bytes = (uint32_t)R * 210;
     uint32_t vw[kLoads];
